@@ -22,7 +22,7 @@ BUILD = os.path.join(HERE, "_build")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
-HIP_SOURCES = ["routing.hip", "align.hip", "elementwise.hip", "moe_gemm.hip",
+HIP_SOURCES = ["routing.hip", "align.hip", "elementwise.hip", "moe_gemm.hip", "moe_gemm_mid.hip",
                "moe_gemm_big.hip", "moe_gemm_pipe.hip", "moe_gemm_stream.hip",
                "moe_gemm_wide.hip", "moe_gemm_wide8.hip", "moe_gemm_wide8p.hip", "moe_gemm_wide4.hip", "moe_gemm_big8.hip", "fused_moe.hip", "prologue.hip", "errors.cpp"]
 HIPCC_FLAGS = [

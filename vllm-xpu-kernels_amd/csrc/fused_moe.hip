@@ -513,7 +513,8 @@ bool stream_khalves_enabled() {
   return !(v && v[0] == '0');
 }
 
-FusedLayout plan(const mi355moe_fused_moe_args* a, uint8_t* base) {
+// max_bm: SMALL blocks of at most that many slots (plan() below)
+FusedLayout plan_with(const mi355moe_fused_moe_args* a, uint8_t* base, int max_bm) {
   FusedLayout L{};
   const int64_t E = a->num_experts;
   L.slots = a->num_tokens * a->topk;
@@ -522,7 +523,16 @@ FusedLayout plan(const mi355moe_fused_moe_args* a, uint8_t* base) {
   const bool kblock = a->w_layout == MI355MOE_WLAYOUT_KBLOCK;
   const bool wide_ok = wide_ok_for(gemm_recipe(a), a->num_tokens, 2 * I, H, kblock) &&
                        wide_ok_for(gemm_recipe(a), L.slots + E * kWideBM, H, K2, kblock);
-  L.tile = pick_tile(gemm_recipe(a), wide_ok, L.slots, E, &L.bm);
+  // expert parallelism: of the slots routed over expert_map_len experts this
+  // rank's E take their share (rank of 8 of DeepSeek-V3, 1003 tokens: 31 slots
+  // per expert, not 251; the 320-slot kernel took 332 us, 64-slot blocks 297)
+  int64_t local = L.slots;
+  if (a->expert_map && a->expert_map_len > E) local = cdiv(L.slots * E, a->expert_map_len);
+  L.tile = pick_tile(gemm_recipe(a), wide_ok, L.slots, local, E, &L.bm);
+  if (L.tile == TILE_SMALL && !(mid_fits(2 * I, H) && mid_fits(H, K2))) {
+    L.tile = TILE_STREAM;  // 64-bit weight offsets
+    L.bm = 16;
+  }
   // K-blocked weights: the families that read them (STREAM, SMALL, WIDE, and
   // BIG for fp8, whose 8-wave kernel takes K <= 8192, and for mxfp4)
   if (kblock && a->recipe != MI355MOE_RECIPE_MXFP4 &&
@@ -531,6 +541,7 @@ FusedLayout plan(const mi355moe_fused_moe_args* a, uint8_t* base) {
     L.tile = TILE_SMALL;
     L.bm = 64;
   }
+  if (L.tile == TILE_SMALL) L.bm = std::min(L.bm, max_bm);
   padded_sizes(L.slots, E, L.bm, L.max_padded, L.max_blocks);
   L.grid_blocks = launch_blocks(L.slots, E, L.bm, L.max_blocks);
   Carver c{base};
@@ -608,6 +619,15 @@ FusedLayout plan(const mi355moe_fused_moe_args* a, uint8_t* base) {
   return L;
 }
 
+// The layer's plan in a workspace of `limit` bytes: where the preferred SMALL
+// blocks pad the activation beyond it, smaller ones.
+FusedLayout plan(const mi355moe_fused_moe_args* a, uint8_t* base, size_t limit = SIZE_MAX) {
+  FusedLayout L = plan_with(a, base, 128);
+  while (L.bytes > limit && L.tile == TILE_SMALL && L.bm > 16)
+    L = plan_with(a, base, L.bm > 64 ? 64 : L.bm / 2);
+  return L;
+}
+
 }  // namespace
 }  // namespace mi355
 
@@ -676,7 +696,7 @@ int scratch_address(hipStream_t stream, void** out) {
 
 extern "C" int mi355moe_fused_moe_noalloc(const mi355moe_fused_moe_args* a, void* stream) {
   if (int rc = validate(a)) return rc;   // before the arguments size anything
-  const size_t need = mi355moe_fused_moe_workspace_size(a);
+  const size_t need = plan(a, nullptr, MI355MOE_NOALLOC_SCRATCH_BYTES).bytes;
   MI_CHECK(need <= MI355MOE_NOALLOC_SCRATCH_BYTES, MI355MOE_ERR_WORKSPACE,
            "fused_moe_noalloc: this call needs " + std::to_string(need) +
                " bytes of scratch, more than the static " +
@@ -799,7 +819,7 @@ int fused_moe_impl(const mi355moe_fused_moe_args* a, void* ws, size_t ws_bytes,
   const int recipe = a->recipe;
   const bool kblock = a->w_layout == MI355MOE_WLAYOUT_KBLOCK;
   if (T == 0) return MI355MOE_OK;
-  FusedLayout L = plan(a, static_cast<uint8_t*>(ws));
+  FusedLayout L = plan(a, static_cast<uint8_t*>(ws), ws_bytes);
   MI_CHECK(ws && ws_bytes >= L.bytes, MI355MOE_ERR_WORKSPACE,
            "workspace too small for fused_moe");
   hipStream_t st = static_cast<hipStream_t>(stream);
@@ -1133,10 +1153,11 @@ struct GGLayout {
   float* as;
   size_t bytes;
 };
-GGLayout gg_plan(int recipe, bool need_quant, int64_t M, int64_t K, int64_t E,
-                 uint8_t* base) {
+GGLayout gg_carve(GemmTile tile, int bm, bool need_quant, int64_t M, int64_t K, int64_t E,
+                  uint8_t* base) {
   GGLayout L{};
-  L.tile = pick_tile(recipe, wide_ok_for(recipe, M, 0, K), M, E, &L.bm);
+  L.tile = tile;
+  L.bm = bm;
   padded_sizes(M, E, L.bm, L.max_padded, L.max_blocks);
   L.grid_blocks = launch_blocks(M, E, L.bm, L.max_blocks);
   Carver c{base};
@@ -1149,8 +1170,24 @@ GGLayout gg_plan(int recipe, bool need_quant, int64_t M, int64_t K, int64_t E,
     L.as = c.take<float>(M * (K / 128));
   }
   L.bytes = c.off + 256;
-  (void)recipe;
   return L;
+}
+GGLayout gg_plan(int recipe, bool need_quant, int64_t M, int64_t N, int64_t K, int64_t E,
+                 uint8_t* base) {
+  int bm;
+  GemmTile tile = pick_tile(recipe, wide_ok_for(recipe, M, 0, K), M, M, E, &bm);
+  if (tile == TILE_SMALL && !mid_fits(N, K)) {
+    tile = TILE_STREAM;  // 64-bit weight offsets
+    bm = 16;
+  }
+  return gg_carve(tile, bm, need_quant, M, K, E, base);
+}
+// bytes that hold the plan of any recipe and N
+size_t gg_bytes(bool need_quant, int64_t M, int64_t K, int64_t E) {
+  size_t most = 0;
+  for (int bm : {16, 32, 64, 96, 128, kWideBM})
+    most = std::max(most, gg_carve(TILE_STREAM, bm, need_quant, M, K, E, nullptr).bytes);
+  return most;
 }
 }  // namespace
 
@@ -1159,7 +1196,7 @@ extern "C" size_t mi355moe_grouped_gemm_workspace_size(int64_t total_rows,
   // worst case: the fp8 recipe quantising a 16-bit A; K is not known here, so
   // callers that pass a 16-bit A to the fp8 recipe must use
   // mi355moe_grouped_gemm_workspace_size_k.
-  return gg_plan(0, false, total_rows, 0, num_experts, nullptr).bytes;
+  return gg_bytes(false, total_rows, 0, num_experts);
 }
 
 extern "C" size_t mi355moe_grouped_gemm_workspace_size_k(int recipe, int a_dtype,
@@ -1167,7 +1204,7 @@ extern "C" size_t mi355moe_grouped_gemm_workspace_size_k(int recipe, int a_dtype
                                                          int64_t K,
                                                          int64_t num_experts) {
   const bool q = recipe == MI355MOE_RECIPE_FP8BLOCK && a_dtype != MI355MOE_FP8E4M3;
-  return gg_plan(recipe, q, total_rows, K, num_experts, nullptr).bytes;
+  return gg_bytes(q, total_rows, K, num_experts);
 }
 
 namespace {
@@ -1220,7 +1257,7 @@ int grouped_gemm_impl(int recipe, const void* A, int a_dtype, const float* a_sca
     MI_ARG(K % 8 == 0, "K must be a multiple of 8");
   }
   if (M == 0) return MI355MOE_OK;
-  GGLayout L = gg_plan(recipe, need_quant, M, K, E, static_cast<uint8_t*>(ws));
+  GGLayout L = gg_plan(recipe, need_quant, M, N, K, E, static_cast<uint8_t*>(ws));
   MI_CHECK(ws && ws_bytes >= L.bytes, MI355MOE_ERR_WORKSPACE,
            "workspace too small for grouped_gemm");
   hipStream_t st = static_cast<hipStream_t>(stream);

@@ -25,11 +25,11 @@ __host__ __device__ constexpr bool is_mx_recipe(int r) {
 __host__ __device__ constexpr bool is_w8a16_recipe(int r) {
   return r == MI355MOE_RECIPE_FP8 || r == MI355MOE_RECIPE_FP8E5M2;
 }
-// 16-bit (and w8a16) weights: layers averaging at most this many slots per
-// active expert run the STREAM kernels, up to kSmallMaxAvg16 the 64-slot
-// SMALL kernels
-constexpr int64_t kStreamMaxAvg16 = 10;
-constexpr int64_t kSmallMaxAvg16 = 48;
+// Layers of at most this many slots run the STREAM kernels: their workgroups
+// route the slots themselves, split K over idle CUs and reduce (gpt-oss-20b,
+// 4 tokens: 64 us, SMALL 68; with more slots SMALL is the faster: DeepSeek-V3,
+// 3 tokens, 226 -> 211 us, Qwen3-30B bf16, 8 tokens, 117 -> 104).
+constexpr int64_t kStreamMaxSlots = 16;
 
 // The split-K w13 GEMM of the fused layer left its partial tiles (no
 // finalize launch); the STREAM w2 launch rebuilds each workgroup's 16-bit
@@ -98,11 +98,6 @@ struct GemmArgs {
   // 64 weight rows (the split gate / up halves of an interleaved swigluoai
   // w13, whose 128-row blocks each held 64 gates and their 64 ups); 0 = 128
   int32_t ws_rows64;
-  // SMALL kernels, order of the (M-block, N-tile) pairs over the XCDs (set
-  // by the launcher): 1 = all N-tiles of an M-block on one XCD, -1 = spread
-  // round-robin, 0 = the first for 16-bit activations averaging 8 or more
-  // valid rows per block, else the second
-  int32_t xcd_order;
   // MX recipes: e8m0 activation scales u8, row r's 32-K group g at
   // a_mxs[r * a_mxs_ld + g] (a_mxs_ld >= K/32; a multiple of 4 where a kernel
   // moves them four at a time); the w13 epilogue of the fused layer writes
@@ -253,35 +248,23 @@ __device__ __forceinline__ void tile_coords(const GemmArgs& a, int t, int n_tile
   }
 }
 
-// Launch over max_blocks M-blocks of bm rows.  bm in {16, 32, 64, 128}.
-int launch_moe_gemm(int recipe, int epi, int bm, const GemmArgs& a,
-                    int64_t max_blocks, hipStream_t st);
-
-// Block size by the expected rows per active expert (16 up to 24, 32 up to
-// 48, 64 up to 96, else 128): the SMALL family's block when forced.
-int pick_block_m(int64_t slots, int64_t num_experts);
-
 // Kernel family and block size by recipe and the expected slots per active
-// expert (avg), break points measured over the benchmark configurations
-// (bf16 Qwen3-30B-A3B, fp8 DeepSeek-V3 and Qwen3-235B, mxfp4 gpt-oss-20b,
-// 1..8192 tokens, every family forced in turn):
-//   bf16   avg <= 10 STREAM;  <= 48 SMALL bm 64;                     else WIDE
-//   fp8    avg <= 4  STREAM;  <= 12 SMALL bm 16;   <= 160 BIG;        else WIDE
-//   mxfp4  avg <= 2  STREAM;  <= 24 SMALL bm 16;   <= 40 SMALL bm 32; else WIDE
-// STREAM: independent-wave weight streaming, 16-slot blocks; SMALL: LDS-shared
-// activation tile; BIG: 128x256 LDS-staged tiles, 128-slot blocks; WIDE:
-// 320x256 tiles, 320-slot blocks (kWideBM), where the shape fits (wide_ok,
-// see wide_ok_for; otherwise bf16 SMALL bm 64 up to avg 96, mxfp4 SMALL bm 32
-// up to 48, then BIG).
-// MI355MOE_GEMM_TILE=stream|small|big|bigreg|wide overrides (A/B
-// measurements; wide falls back to big where it does not apply, small takes
-// pick_block_m's block size).
+// expert (avg): at most kStreamMaxSlots slots in the call STREAM (16-slot blocks,
+// independent waves); then SMALL (small_block in moe_gemm.hip has the block
+// sizes, the ends of its range and the measurements); beyond it WIDE (320x256
+// tiles, 320-slot blocks) where the shape fits (wide_ok, see wide_ok_for),
+// else BIG (128x256 LDS-staged tiles, 128-slot blocks).  The MX recipes run
+// WIDE from 17 slots per expert on, STREAM below.
+// MI355MOE_GEMM_TILE=stream|small|big|bigreg|wide overrides (tests, A/B
+// measurements; wide falls back to big where it does not apply).
 // (TILE_BIG runs the 8-wave fp8 kernel where big8_supported(), else the
 // LDS-DMA pipelined kernel where pipe_supported(), else the register-staged
 // one, which TILE_BIGREG forces.)
 enum GemmTile { TILE_STREAM = 0, TILE_SMALL = 1, TILE_BIG = 2, TILE_BIGREG = 3, TILE_WIDE = 4 };
 constexpr int kWideBM = 320;  // slots per block of the WIDE family
-GemmTile pick_tile(int recipe, bool wide_ok, int64_t slots, int64_t num_experts, int* bm);
+// slots: all of the call's; local: those expected on this rank's experts.
+GemmTile pick_tile(int recipe, bool wide_ok, int64_t slots, int64_t local, int64_t num_experts,
+                   int* bm);
 // Whether a GEMM with a_rows activation rows, ldb_rows weight rows per
 // expert (0: not known yet), reduction length K and the given weight layout
 // fits the WIDE kernels (mxfp4: K-blocked weights only).
@@ -292,8 +275,11 @@ int launch_tile_gemm(GemmTile tile, int bm, int recipe, int epi, bool qout,
                      const GemmArgs& a, int64_t max_blocks, void* qs,
                      hipStream_t st);
 
-int launch_moe_gemm_q(int recipe, int epi, bool qout, int bm, const GemmArgs& a,
-                      int64_t max_blocks, void* qs, hipStream_t st);
+// Blocks of bm (16, 32, 64, 96 or 128) slots, every recipe but the MX ones
+// (moe_gemm_mid.hip), for experts of fewer than 2^30 weights (mid_fits).
+bool mid_fits(int64_t ldb_rows, int64_t K);
+int launch_moe_gemm_mid(int recipe, int epi, bool qout, int bm, const GemmArgs& a,
+                        int64_t max_blocks, void* qs, hipStream_t st);
 // 128-slot blocks; GLU tiles cover 128 output columns, STORE tiles 256.
 int launch_moe_gemm_big(int recipe, int epi, bool qout, const GemmArgs& a,
                         int64_t max_blocks, void* qs, hipStream_t st);
