@@ -1,7 +1,7 @@
 // Token -> expert alignment: a deterministic, stable counting sort of the
 // flattened top-k expert ids.  Up to kOneBlockMax ids it runs in one
 // 1024-thread workgroup (one launch, the decode case); larger inputs use
-// three launches over 1024-id chunks (count, scan, scatter) with the same
+// two launches over 1024-id chunks (count; scan and scatter) with the same
 // ordering rule, so that the scattered stores of the sorted ids spread over
 // the whole GPU instead of one CU.
 //
@@ -9,10 +9,16 @@
 // "chunk order, then rank inside the chunk" is flat order.  Per-chunk expert
 // counts live in LDS (16 x E ints); a block-wide scan turns them into each
 // chunk's first output slot per expert; the scatter pass ranks the lanes of
-// every 64-element step that carry the same expert with 11 ballots (one per
-// key bit), so no atomics decide the order.  Replaces the reference's
+// every 64-element step that carry the same expert with one ballot per key
+// bit, so no atomics decide the order.  Replaces the reference's
 // count + device-atomic scatter (csrc/moe/moe_align_sum_kernels.cpp:135-455),
 // whose within-expert order is not deterministic.
+//
+// Both forms are chains of latencies (id load, LDS counts, scan, scatter):
+// what counts is the number of round trips and launches.  The multi-workgroup
+// form took three launches (5 + 5 + 17 us for 24008 ids of 128 experts, 320-id
+// blocks), its scatter most of that time finding the expert of every padding
+// position by binary search.
 #include <type_traits>
 
 #include "common.h"
@@ -25,6 +31,7 @@ constexpr int kSortThreads = 1024;
 constexpr int kSortWaves = kSortThreads / 64;
 constexpr int kMaxKeys = 1024;
 constexpr uint32_t kInvalidKey = 2047u;  // 11 bits, never a valid key
+constexpr int kOneBlockMax = 4096;  // ids one workgroup sorts
 
 // Options of the fused_moe_prologue sort: ids are shifted by `start` (the
 // rank's first expert); with dedupe_k > 1 a slot whose token chose the same
@@ -87,6 +94,58 @@ __device__ int block_exclusive_scan(int v, int* s_wave_tot, int& total) {
   return before + x - v;
 }
 
+// Bits that tell the keys 0 .. num_keys - 1 and kInvalidKey (all ones) apart.
+__device__ __forceinline__ int key_bits(int num_keys) { return 32 - __clz(num_keys); }
+
+// Output slot of this lane's key: the wave's next slot of that key (cnt,
+// advanced past the wave's ids of it) plus the lanes below with the same key;
+// -1 for kInvalidKey.  All 64 lanes must be active.
+__device__ __forceinline__ int place(uint32_t key, int bits, int lane, int* cnt) {
+  unsigned long long same = ~0ull;
+  for (int b = 0; b < bits; ++b) {
+    const unsigned long long bb = __ballot((key >> b) & 1u);
+    same &= ((key >> b) & 1u) ? bb : ~bb;
+  }
+  const int rank = __popcll(same & ((1ull << lane) - 1ull));
+  int pos = -1;
+  if (key != kInvalidKey) {
+    pos = cnt[key] + rank;
+    if (rank == 0) cnt[key] += __popcll(same);
+  }
+  return pos;
+}
+
+// The padding slots of every expert's range, its blocks' expert ids, and
+// (not keep_tail) what follows the padded total; wave w of nw takes experts w,
+// w + nw, ..., thread t of nt the tails.
+__device__ __forceinline__ void write_padding(const int* s_cum, const int* s_tot, int num_keys,
+                                              int block_size, int32_t* __restrict__ sorted_ids,
+                                              int64_t max_padded,
+                                              int32_t* __restrict__ expert_ids,
+                                              int64_t max_blocks, int32_t pad_value,
+                                              int32_t no_expert, bool keep_tail, int w, int nw,
+                                              int t, int nt) {
+  const int lane = threadIdx.x & 63;
+  for (int e = w; e < num_keys; e += nw) {
+    const int start = s_cum[e], end = s_cum[e + 1];
+    if (sorted_ids)
+      for (int p = start + s_tot[e] + lane; p < end && p < max_padded; p += 64)
+        sorted_ids[p] = pad_value;
+    if (expert_ids) {
+      const int b1 = end / block_size;
+      for (int b = start / block_size + lane; b < b1 && b < max_blocks; b += 64)
+        expert_ids[b] = e;
+    }
+  }
+  const int total = s_cum[num_keys];
+  if (sorted_ids && !keep_tail)
+    for (int64_t p = static_cast<int64_t>(total) + t; p < max_padded; p += nt)
+      sorted_ids[p] = pad_value;
+  if (expert_ids)
+    for (int64_t b = static_cast<int64_t>(total / block_size) + t; b < max_blocks; b += nt)
+      expert_ids[b] = no_expert;
+}
+
 // Multi-LoRA alignment (moe_lora_align_block_size): workgroup w sorts, for
 // the adapter lora_ids[w], only the slots of tokens mapped to it, into its own
 // slices of the outputs; invalid (-1, >= max_loras) or disabled adapters
@@ -110,6 +169,7 @@ __device__ __forceinline__ void counting_sort_body(
     int32_t pad_value, LoraSel lora, KeyXform xf) {
   __shared__ int s_cnt[kSortWaves][kMaxKeys];
   __shared__ int s_cum[kMaxKeys + 1];
+  __shared__ int s_tot[kMaxKeys];
   __shared__ int s_wave_tot[kSortWaves];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int lora_id = 0;
@@ -129,41 +189,58 @@ __device__ __forceinline__ void counting_sort_body(
     return key;
   };
 
-  for (int i = tid; i < kSortWaves * kMaxKeys; i += kSortThreads)
-    (&s_cnt[0][0])[i] = 0;
-  __syncthreads();
-
   const int64_t chunk = ((numel + kSortWaves - 1) / kSortWaves + 63) / 64 * 64;
   const int64_t lo = wave * chunk;
   const int64_t hi = lo + chunk < numel ? lo + chunk : numel;
   const int steps = static_cast<int>(chunk / 64);
+  // the first steps' keys stay in registers (all of them up to kOneBlockMax
+  // ids), loaded together while the counters are cleared
+  constexpr int kRegSteps = kOneBlockMax / kSortThreads;
+  uint32_t keys[kRegSteps];
+#pragma unroll
+  for (int s = 0; s < kRegSteps; ++s) {
+    const int64_t i = lo + static_cast<int64_t>(s) * 64 + lane;
+    keys[s] = s < steps && i < hi ? key_of(i) : kInvalidKey;
+  }
+  for (int w = 0; w < kSortWaves; ++w)
+    if (tid < num_keys) s_cnt[w][tid] = 0;
+  __syncthreads();
 
   // phase 1: per-chunk counts
-  for (int s = 0; s < steps; ++s) {
-    int64_t i = lo + static_cast<int64_t>(s) * 64 + lane;
+#pragma unroll
+  for (int s = 0; s < kRegSteps; ++s)
+    if (keys[s] != kInvalidKey) atomicAdd(&s_cnt[wave][keys[s]], 1);
+  for (int s = kRegSteps; s < steps; ++s) {
+    const int64_t i = lo + static_cast<int64_t>(s) * 64 + lane;
     if (i < hi) {
-      uint32_t key = key_of(i);
+      const uint32_t key = key_of(i);
       if (key != kInvalidKey) atomicAdd(&s_cnt[wave][key], 1);
     }
   }
   __syncthreads();
 
-  // phase 2: per-expert totals, chunk-exclusive offsets, padded scan
+  // phase 2: per-expert totals, padded scan, first slot of every chunk
+  int c[kSortWaves];
   int total_e = 0;
   if (tid < num_keys) {
-    for (int w = 0; w < kSortWaves; ++w) {
-      int c = s_cnt[w][tid];
-      s_cnt[w][tid] = total_e;
-      total_e += c;
-    }
+#pragma unroll
+    for (int w = 0; w < kSortWaves; ++w) c[w] = s_cnt[w][tid];
+#pragma unroll
+    for (int w = 0; w < kSortWaves; ++w) total_e += c[w];
   }
   const int padded = (total_e + block_size - 1) / block_size * block_size;
   int total_padded = 0;
   const int start = block_exclusive_scan(tid < num_keys ? padded : 0,
                                          s_wave_tot, total_padded);
   if (tid < num_keys) {
+    int run = start;
+#pragma unroll
+    for (int w = 0; w < kSortWaves; ++w) {
+      s_cnt[w][tid] = run;
+      run += c[w];
+    }
     s_cum[tid] = start;
-    for (int w = 0; w < kSortWaves; ++w) s_cnt[w][tid] += start;
+    s_tot[tid] = total_e;
     if (counts_out) counts_out[tid] = total_e;
     if (cum_out) cum_out[tid] = start;
   }
@@ -174,58 +251,26 @@ __device__ __forceinline__ void counting_sort_body(
   }
   __syncthreads();
 
-  // padding slots inside each expert's range and the tail
-  if (sorted_ids) {
-    if (tid < num_keys) {
-      for (int p = start + total_e; p < start + padded && p < max_padded; ++p)
-        sorted_ids[p] = pad_value;
-    }
-    if (!xf.keep_tail)
-      for (int64_t p = total_padded + tid; p < max_padded; p += kSortThreads)
-        sorted_ids[p] = pad_value;
-  }
-  // expert id of every block (binary search over the padded prefix)
-  if (expert_ids) {
-    const int nblk = total_padded / block_size;
-    for (int64_t b = tid; b < max_blocks; b += kSortThreads) {
-      int e = 0;
-      if (b < nblk) {
-        int lo_e = 0, hi_e = num_keys - 1;
-        const int p = static_cast<int>(b) * block_size;
-        while (lo_e < hi_e) {  // last e with s_cum[e] <= p
-          int mid = (lo_e + hi_e + 1) >> 1;
-          if (s_cum[mid] <= p) lo_e = mid; else hi_e = mid - 1;
-        }
-        e = lo_e;
-      }
-      expert_ids[b] = b < nblk ? e : (LORA ? -1 : 0);
-    }
+  // phase 3: stable scatter (a wave's counters are its own, and the LDS
+  // accesses of one wave execute in program order)
+  const int bits = key_bits(num_keys);
+  auto step = [&](int s, uint32_t key) {
+    const int64_t i = lo + static_cast<int64_t>(s) * 64 + lane;
+    const int pos = place(key, bits, lane, s_cnt[wave]);
+    if (pos >= 0 && sorted_ids && pos < max_padded) sorted_ids[pos] = static_cast<int32_t>(i);
+    if (inv_pos && i < hi) inv_pos[inv_index(i, xf)] = pos;
+  };
+#pragma unroll
+  for (int s = 0; s < kRegSteps; ++s)
+    if (s < steps) step(s, keys[s]);
+  for (int s = kRegSteps; s < steps; ++s) {
+    const int64_t i = lo + static_cast<int64_t>(s) * 64 + lane;
+    step(s, i < hi ? key_of(i) : kInvalidKey);
   }
 
-  // phase 3: stable scatter
-  const unsigned long long below = (1ull << lane) - 1ull;
-  for (int s = 0; s < steps; ++s) {
-    int64_t i = lo + static_cast<int64_t>(s) * 64 + lane;
-    uint32_t key = kInvalidKey;
-    if (i < hi) key = key_of(i);
-    unsigned long long same = ~0ull;
-#pragma unroll
-    for (int b = 0; b < 11; ++b) {
-      unsigned long long bb = __ballot((key >> b) & 1u);
-      same &= ((key >> b) & 1u) ? bb : ~bb;
-    }
-    const int rank = __popcll(same & below);
-    const int cnt = __popcll(same);
-    int pos = -1;
-    if (key != kInvalidKey) {
-      pos = s_cnt[wave][key] + rank;
-      if (sorted_ids && pos < max_padded) sorted_ids[pos] = static_cast<int32_t>(i);
-    }
-    if (inv_pos && i < hi) inv_pos[inv_index(i, xf)] = pos;
-    __syncthreads();
-    if (key != kInvalidKey && rank == 0) s_cnt[wave][key] += cnt;
-    __syncthreads();
-  }
+  write_padding(s_cum, s_tot, num_keys, block_size, sorted_ids, max_padded, expert_ids,
+                max_blocks, pad_value, LORA ? -1 : 0, xf.keep_tail, wave, kSortWaves, tid,
+                kSortThreads);
 }
 
 template <typename Id, bool LORA = false>
@@ -258,7 +303,7 @@ __global__ __launch_bounds__(kSortThreads) void sort_quant_kernel(
   if (blockIdx.x == 0) {
     counting_sort_body<Id, false>(ids, numel, id_bound, map, num_keys, block_size, sorted_ids,
                                   max_padded, expert_ids, max_blocks, ntp, inv_pos, nullptr,
-                                  cum_out, pad_value, LoraSel{}, KeyXform{});
+                                  cum_out, pad_value, LoraSel{}, KeyXform{0, 0, true, 0});
     return;
   }
   fp8_quant_block8<F16>(x, xq, xs, (static_cast<int64_t>(blockIdx.x) - 1) * kSortThreads +
@@ -267,178 +312,146 @@ __global__ __launch_bounds__(kSortThreads) void sort_quant_kernel(
 
 // ---------------------------------------------------------------------------
 // Multi-workgroup sort.  Chunk c holds ids [c*chunk, (c+1)*chunk); chunk is a
-// multiple of 256 so each of a chunk's 4 waves owns a contiguous multiple of
+// multiple of 1024 so each of a chunk's 16 waves owns a contiguous multiple of
 // 64 ids.  "chunk order, wave order, rank inside the 64-id step" is flat
 // order, as in the one-workgroup kernel.
-constexpr int kOneBlockMax = 4096;
 constexpr int kChunkIds = 1024;
 constexpr int kMaxChunks = 1024;
 
 inline int64_t sort_chunk(int64_t numel) {
   int64_t c = cdiv(numel, kChunkIds);
   if (c > kMaxChunks) c = kMaxChunks;
-  return cdiv(cdiv(numel, c), 256) * 256;
+  return cdiv(cdiv(numel, c), kSortThreads) * kSortThreads;
 }
 
 // per-chunk expert counts: cnt[c][e]
 template <typename Id>
-__global__ __launch_bounds__(256) void chunk_count_kernel(
+__global__ __launch_bounds__(kSortThreads) void chunk_count_kernel(
     const Id* __restrict__ ids, int64_t numel, int64_t id_bound,
     const int32_t* __restrict__ map, int num_keys, int64_t chunk,
     int32_t* __restrict__ cnt, KeyXform xf) {
   __shared__ int s[kMaxKeys];
-  for (int e = threadIdx.x; e < num_keys; e += 256) s[e] = 0;
+  const int tid = threadIdx.x;
+  if (tid < num_keys) s[tid] = 0;
   __syncthreads();
   const int64_t lo = static_cast<int64_t>(blockIdx.x) * chunk;
   const int64_t hi = lo + chunk < numel ? lo + chunk : numel;
-  for (int64_t i = lo + threadIdx.x; i < hi; i += 256) {
+  for (int64_t i = lo + tid; i < hi; i += kSortThreads) {
     const uint32_t key = load_key(ids, i, id_bound, map, num_keys, xf);
     if (key != kInvalidKey) atomicAdd(&s[key], 1);
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < num_keys; e += 256)
-    cnt[static_cast<int64_t>(blockIdx.x) * num_keys + e] = s[e];
+  if (tid < num_keys) cnt[static_cast<int64_t>(blockIdx.x) * num_keys + tid] = s[tid];
 }
 
-// cnt[c][e] -> ids of expert e in chunks before c; cum[e] = padded start of
-// expert e (cum[num_keys] = total padded), tot[e] = its id count.  The
-// chunk counts are read 8 at a time so the loads overlap.
-__global__ __launch_bounds__(kSortThreads) void chunk_scan_kernel(
-    int32_t* __restrict__ cnt, int nchunks, int num_keys, int block_size,
-    int32_t* __restrict__ cum, int32_t* __restrict__ tot,
-    int32_t* __restrict__ ntp, int32_t* __restrict__ counts_out,
-    int32_t* __restrict__ cum_out) {
-  __shared__ int s_wave_tot[kSortWaves];
-  const int tid = threadIdx.x;
-  int total_e = 0;
-  if (tid < num_keys) {
-    for (int c0 = 0; c0 < nchunks; c0 += 8) {
-      int v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        v[u] = c0 + u < nchunks ? cnt[static_cast<int64_t>(c0 + u) * num_keys + tid] : 0;
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        if (c0 + u < nchunks) cnt[static_cast<int64_t>(c0 + u) * num_keys + tid] = total_e;
-        total_e += v[u];
-      }
-    }
-  }
-  const int padded = (total_e + block_size - 1) / block_size * block_size;
-  int total_padded = 0;
-  const int start = block_exclusive_scan(tid < num_keys ? padded : 0, s_wave_tot,
-                                         total_padded);
-  if (tid < num_keys) {
-    cum[tid] = start;
-    tot[tid] = total_e;
-    if (counts_out) counts_out[tid] = total_e;
-    if (cum_out) cum_out[tid] = start;
-  }
-  if (tid == 0) {
-    cum[num_keys] = total_padded;
-    if (ntp) ntp[0] = total_padded;
-    if (cum_out) cum_out[num_keys] = total_padded;
-  }
-}
-
-// Stable scatter of chunk blockIdx.x, then (grid-strided) the padding slots,
-// the tail past the padded total and the expert id of every block.
+// Every workgroup sums the chunks' counts for itself (totals, and those of
+// the chunks before its own), which saves a scan launch; then the stable
+// scatter of chunk blockIdx.x and a share of the padding.
 template <typename Id>
-__global__ __launch_bounds__(256) void chunk_scatter_kernel(
+__global__ __launch_bounds__(kSortThreads) void chunk_scatter_kernel(
     const Id* __restrict__ ids, int64_t numel, int64_t id_bound,
     const int32_t* __restrict__ map, int num_keys, int64_t chunk,
-    const int32_t* __restrict__ off, const int32_t* __restrict__ cum,
-    const int32_t* __restrict__ tot, int block_size,
+    const int32_t* __restrict__ cnt, int nchunks, int block_size,
     int32_t* __restrict__ sorted_ids, int64_t max_padded,
     int32_t* __restrict__ expert_ids, int64_t max_blocks,
-    int32_t* __restrict__ inv_pos, int32_t pad_value, KeyXform xf) {
-  __shared__ int s_cnt[4][kMaxKeys];
+    int32_t* __restrict__ ntp, int32_t* __restrict__ inv_pos,
+    int32_t* __restrict__ counts_out, int32_t* __restrict__ cum_out,
+    int32_t pad_value, KeyXform xf) {
+  __shared__ int s_cnt[kSortWaves][kMaxKeys];
   __shared__ int s_cum[kMaxKeys + 1];
   __shared__ int s_tot[kMaxKeys];
+  __shared__ int s_before[kMaxKeys];
+  __shared__ int s_wave_tot[kSortWaves];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  for (int i = tid; i < 4 * kMaxKeys; i += 256) (&s_cnt[0][0])[i] = 0;
-  for (int e = tid; e <= num_keys; e += 256) {
-    s_cum[e] = cum[e];
-    if (e < num_keys) s_tot[e] = tot[e];
-  }
-  __syncthreads();
-
-  const int64_t sub = chunk / 4;
-  const int64_t clo = static_cast<int64_t>(blockIdx.x) * chunk;
-  const int64_t lo = clo + wave * sub;
+  const int me = static_cast<int>(blockIdx.x);
+  const int64_t sub = chunk / kSortWaves;
+  const int64_t lo = static_cast<int64_t>(me) * chunk + wave * sub;
   const int64_t hi0 = lo + sub < numel ? lo + sub : numel;
   const int64_t hi = hi0 > lo ? hi0 : lo;
   const int steps = static_cast<int>(sub / 64);
-  for (int s = 0; s < steps; ++s) {
+  // the first step's keys (all of them up to a million ids) stay in a register
+  const uint32_t key0 = lo + lane < hi ? load_key(ids, lo + lane, id_bound, map, num_keys, xf)
+                                       : kInvalidKey;
+  for (int w = 0; w < kSortWaves; ++w)
+    if (tid < num_keys) s_cnt[w][tid] = 0;
+  if (tid < num_keys) s_tot[tid] = s_before[tid] = 0;
+  __syncthreads();
+
+  if (key0 != kInvalidKey) atomicAdd(&s_cnt[wave][key0], 1);
+  for (int s = 1; s < steps; ++s) {
     const int64_t i = lo + static_cast<int64_t>(s) * 64 + lane;
     if (i < hi) {
       const uint32_t key = load_key(ids, i, id_bound, map, num_keys, xf);
       if (key != kInvalidKey) atomicAdd(&s_cnt[wave][key], 1);
     }
   }
-  __syncthreads();
-  // wave w's first slot for expert e: expert start + ids in earlier chunks
-  // + ids of waves < w
-  for (int e = tid; e < num_keys; e += 256) {
-    int run = s_cum[e] + off[static_cast<int64_t>(blockIdx.x) * num_keys + e];
+  // thread group g takes chunks g, g + G, ... of key tid % stride, eight
+  // loads in flight; integer LDS sums, so their order does not matter
+  {
+    const int stride = 1 << key_bits(num_keys - 1);
+    const int G = kSortThreads / stride, g = tid / stride, e = tid % stride;
+    if (g < G && e < num_keys) {
+      int total = 0, before = 0;
+      for (int c0 = g; c0 < nchunks; c0 += 8 * G) {
+        int v[8];
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const int c = s_cnt[w][e];
-      s_cnt[w][e] = run;
-      run += c;
+        for (int u = 0; u < 8; ++u) {
+          const int c = c0 + u * G;
+          v[u] = c < nchunks ? cnt[static_cast<int64_t>(c) * num_keys + e] : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          total += v[u];
+          before += c0 + u * G < me ? v[u] : 0;
+        }
+      }
+      atomicAdd(&s_tot[e], total);
+      atomicAdd(&s_before[e], before);
     }
   }
   __syncthreads();
-  // each wave ranks its own 64-id steps; its counters are its own, and the
-  // LDS accesses of one wave execute in program order
-  const unsigned long long below = (1ull << lane) - 1ull;
+  const int total_e = tid < num_keys ? s_tot[tid] : 0;
+  const int padded = (total_e + block_size - 1) / block_size * block_size;
+  int total_padded = 0;
+  const int start = block_exclusive_scan(tid < num_keys ? padded : 0, s_wave_tot, total_padded);
+  if (tid < num_keys) {
+    // wave w's first slot: expert start + ids in earlier chunks + ids of waves < w
+    int c[kSortWaves];
+#pragma unroll
+    for (int w = 0; w < kSortWaves; ++w) c[w] = s_cnt[w][tid];
+    int run = start + s_before[tid];
+#pragma unroll
+    for (int w = 0; w < kSortWaves; ++w) {
+      s_cnt[w][tid] = run;
+      run += c[w];
+    }
+    s_cum[tid] = start;
+    if (me == 0) {
+      if (counts_out) counts_out[tid] = total_e;
+      if (cum_out) cum_out[tid] = start;
+    }
+  }
+  if (tid == 0) {
+    s_cum[num_keys] = total_padded;
+    if (me == 0) {
+      if (ntp) ntp[0] = total_padded;
+      if (cum_out) cum_out[num_keys] = total_padded;
+    }
+  }
+  __syncthreads();
+  const int bits = key_bits(num_keys);
   for (int s = 0; s < steps; ++s) {
     const int64_t i = lo + static_cast<int64_t>(s) * 64 + lane;
-    uint32_t key = kInvalidKey;
-    if (i < hi) key = load_key(ids, i, id_bound, map, num_keys, xf);
-    unsigned long long same = ~0ull;
-#pragma unroll
-    for (int b = 0; b < 11; ++b) {
-      const unsigned long long bb = __ballot((key >> b) & 1u);
-      same &= ((key >> b) & 1u) ? bb : ~bb;
-    }
-    const int rank = __popcll(same & below);
-    const int cnt = __popcll(same);
-    int pos = -1;
-    if (key != kInvalidKey) {
-      pos = s_cnt[wave][key] + rank;
-      if (sorted_ids && pos < max_padded) sorted_ids[pos] = static_cast<int32_t>(i);
-    }
+    uint32_t key = key0;
+    if (s > 0) key = i < hi ? load_key(ids, i, id_bound, map, num_keys, xf) : kInvalidKey;
+    const int pos = place(key, bits, lane, s_cnt[wave]);
+    if (pos >= 0 && sorted_ids && pos < max_padded) sorted_ids[pos] = static_cast<int32_t>(i);
     if (inv_pos && i < hi) inv_pos[inv_index(i, xf)] = pos;
-    if (key != kInvalidKey && rank == 0) s_cnt[wave][key] += cnt;
   }
-
-  // padding slots of every expert and the tail, expert id of every block
-  const int total_padded = s_cum[num_keys];
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
-  auto expert_at = [&](int p) -> int {  // last e with s_cum[e] <= p
-    int lo_e = 0, hi_e = num_keys - 1;
-    while (lo_e < hi_e) {
-      const int mid = (lo_e + hi_e + 1) >> 1;
-      if (s_cum[mid] <= p) lo_e = mid; else hi_e = mid - 1;
-    }
-    return lo_e;
-  };
-  if (sorted_ids) {
-    for (int64_t p = static_cast<int64_t>(blockIdx.x) * 256 + tid; p < max_padded; p += stride) {
-      if (p >= total_padded) {
-        if (!xf.keep_tail) sorted_ids[p] = pad_value;
-      } else {
-        const int e = expert_at(static_cast<int>(p));
-        if (p - s_cum[e] >= s_tot[e]) sorted_ids[p] = pad_value;
-      }
-    }
-  }
-  if (expert_ids) {
-    const int nblk = total_padded / block_size;
-    for (int64_t b = static_cast<int64_t>(blockIdx.x) * 256 + tid; b < max_blocks; b += stride)
-      expert_ids[b] = b < nblk ? expert_at(static_cast<int>(b) * block_size) : 0;
-  }
+  const int wgs = static_cast<int>(gridDim.x);
+  write_padding(s_cum, s_tot, num_keys, block_size, sorted_ids, max_padded, expert_ids,
+                max_blocks, pad_value, 0, xf.keep_tail, me * kSortWaves + wave,
+                wgs * kSortWaves, me * kSortThreads + tid, wgs * kSortThreads);
 }
 
 // rows_per_expert (contiguous segments) -> block-padded row list:
@@ -543,16 +556,11 @@ void launch_sort(const void* ids, int64_t numel, int64_t id_bound,
   }
   const int64_t chunk = sort_chunk(numel);
   const int nchunks = static_cast<int>(cdiv(numel, chunk));
-  int32_t* cnt = ws;
-  int32_t* cum = cnt + static_cast<int64_t>(nchunks) * num_keys;
-  int32_t* tot = cum + num_keys + 1;
-  chunk_count_kernel<Id><<<nchunks, 256, 0, st>>>(id, numel, id_bound, map,
-                                                   num_keys, chunk, cnt, xf);
-  chunk_scan_kernel<<<1, kSortThreads, 0, st>>>(cnt, nchunks, num_keys, bs, cum,
-                                                tot, ntp, counts, cum_out);
-  chunk_scatter_kernel<Id><<<nchunks, 256, 0, st>>>(
-      id, numel, id_bound, map, num_keys, chunk, cnt, cum, tot, bs, sorted,
-      max_padded, eids, max_blocks, inv, pad, xf);
+  chunk_count_kernel<Id><<<nchunks, kSortThreads, 0, st>>>(id, numel, id_bound, map, num_keys,
+                                                           chunk, ws, xf);
+  chunk_scatter_kernel<Id><<<nchunks, kSortThreads, 0, st>>>(
+      id, numel, id_bound, map, num_keys, chunk, ws, nchunks, bs, sorted, max_padded, eids,
+      max_blocks, ntp, inv, counts, cum_out, pad, xf);
 }
 
 }  // namespace
@@ -561,7 +569,7 @@ void launch_sort(const void* ids, int64_t numel, int64_t id_bound,
 size_t counting_sort_ws_bytes(int64_t numel, int64_t num_keys) {
   if (numel <= kOneBlockMax || num_keys <= 0) return 0;
   const int64_t nchunks = cdiv(numel, sort_chunk(numel));
-  return static_cast<size_t>(nchunks * num_keys + 2 * num_keys + 1) * sizeof(int32_t);
+  return static_cast<size_t>(nchunks * num_keys) * sizeof(int32_t);
 }
 
 // Shared by the fused layer and the alignment entry points.  ws: at least
@@ -572,9 +580,9 @@ int run_counting_sort(const void* ids, int ids_dtype, int64_t numel,
                       int32_t* eids, int64_t max_blocks, int32_t* ntp,
                       int32_t* inv, int32_t* counts, int32_t pad,
                       void* ws, size_t ws_bytes, hipStream_t st, int32_t* cum_out,
-                      int64_t id_start, int dedupe_k, int64_t inv_rows) {
+                      int64_t id_start, int dedupe_k, int64_t inv_rows, bool keep_tail) {
   // the prologue's sort (dedupe_k > 0) writes only the sorted slots
-  const KeyXform xf{id_start, dedupe_k, dedupe_k > 0, dedupe_k > 0 ? inv_rows : 0};
+  const KeyXform xf{id_start, dedupe_k, dedupe_k > 0 || keep_tail, dedupe_k > 0 ? inv_rows : 0};
   MI_ARG(num_keys > 0 && num_keys <= kMaxKeys,
          "padded_num_experts must be less than 1024");
   MI_ARG(bs > 0, "block_size must be positive");

@@ -327,7 +327,8 @@ size_t counting_sort_ws_bytes(int64_t numel, int64_t num_keys);
 // only the first occurrence of an expert among a token's dedupe_k ids is
 // kept, sorted entries past the last sorted slot are left as they were, and
 // with inv_rows > 0 the position of slot t * dedupe_k + j goes to
-// inv[j * inv_rows + t].
+// inv[j * inv_rows + t].  keep_tail leaves the entries past the padded total
+// as they are (no GEMM block reads them).
 int run_counting_sort(const void* ids, int ids_dtype, int64_t numel,
                       int64_t id_bound, const int32_t* map, int64_t num_keys,
                       int64_t bs, int32_t* sorted, int64_t max_padded,
@@ -335,7 +336,7 @@ int run_counting_sort(const void* ids, int ids_dtype, int64_t numel,
                       int32_t* inv, int32_t* counts, int32_t pad,
                       void* ws, size_t ws_bytes, hipStream_t st,
                       int32_t* cum_out = nullptr, int64_t id_start = 0,
-                      int dedupe_k = 0, int64_t inv_rows = 0);
+                      int dedupe_k = 0, int64_t inv_rows = 0, bool keep_tail = false);
 // The one-workgroup sort and the e4m3 1 x 128 quantisation of x [rows, cols]
 // (16-bit, f16 or bf16) in one launch (align.hip).  Returns 1 without
 // launching when the sort needs more than one workgroup or x does not fit
