@@ -189,7 +189,7 @@ __global__ __launch_bounds__(512) void moe_gemm_wide_kernel(const GemmArgs a) {
     s_drow[tid] = ok ? (a.d_by_pos ? blk * BM + tid : rid) : -1;
   }
   // valid slots form a prefix of the block
-  const int v = __syncthreads_count(ok);
+  const int v = __builtin_amdgcn_readfirstlane(__syncthreads_count(ok));
 
   // weight row staged at tile row r; rows past N read row 0 (finite data
   // whose outputs are never stored).  GLU: rows [0,128) gate, [128,256) up.
@@ -240,9 +240,12 @@ __global__ __launch_bounds__(512) void moe_gemm_wide_kernel(const GemmArgs a) {
   // LDS block of src[0]
   const uint32_t dst0 = a_wave ? A_DMA * wave * 1024 : A_BYTES + W_DMA * (wave - 4) * 1024;
 
-  // per-wave MFMA rows: 160 wm + [0, 32 nj)
-  const int vw = v - 32 * MG * wm;
-  const int nj = vw <= 0 ? 0 : (vw >= 32 * MG ? MG : (vw + 31) / 32);
+  // per-wave MFMA rows: rbase + [0, 32 nj), the block's 32-row groups split
+  // evenly over the two wave halves (both share each SIMD: a half with all of
+  // them leaves the other idle while it waits for LDS)
+  const int ng = (v + 31) / 32, ng0 = (ng + 1) / 2;
+  const int nj = wm ? ng - ng0 : ng0;
+  const int rbase = wm ? 32 * ng0 : 0;
 
   // fragment offsets within a stage: chunk c = 2 ks + h; every row this lane
   // reads (l32 plus a multiple of 32) has the swizzle of l32
@@ -251,7 +254,7 @@ __global__ __launch_bounds__(512) void moe_gemm_wide_kernel(const GemmArgs a) {
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks) {
     const int c = (2 * ks + h) ^ swz(l32);
-    xoff[ks] = (32 * MG * wm + l32) * ROWB + (c << 4);
+    xoff[ks] = (rbase + l32) * ROWB + (c << 4);
     woff[ks] = A_BYTES + ((kGlu ? 32 * wn : 64 * wn) + l32) * ROWB + (c << 4);
   }
 
@@ -324,10 +327,9 @@ __global__ __launch_bounds__(512) void moe_gemm_wide_kernel(const GemmArgs a) {
 
   // ---- epilogue: bias, rounding, activation; output tile staged in LDS and
   //      written with 16-byte row-contiguous stores (STORE tiles in two
-  //      passes of 160 rows, one per wave half)
+  //      passes, one per wave half)
   constexpr int PITCH = 2 * NOUT + 16;
   constexpr int PASSES = BM * PITCH <= RING_BYTES ? 1 : 2;
-  constexpr int PROWS = BM / PASSES;
   const int64_t bias_base = static_cast<int64_t>(e) * a.ldb_rows;
   const float es = a.expert_scale ? a.expert_scale[e] : 1.f;  // recipe BF16 only
   auto tcol = [&](int i, int r) -> int {  // tile output column of (i, r)
@@ -338,11 +340,11 @@ __global__ __launch_bounds__(512) void moe_gemm_wide_kernel(const GemmArgs a) {
   const bool vec = (N & 7) == 0 && (reinterpret_cast<uintptr_t>(a.D) & 15) == 0;
   constexpr int CPR = 2 * NOUT / 16;  // 16-byte chunks per row
   __syncthreads();  // every wave is done with the ring
-  // the tile's 16-bit outputs into the LDS staging rows of pass `pass`,
+  // the tile's 16-bit outputs into the LDS staging rows,
   // specialised on the activation, gemm1_clamp_limit and the bias (uniform
   // per launch) so that no value branches on them; gate and up rounded two
   // values per conversion
-  auto stage_out = [&](int pass, auto silu_c, auto clamp_c, auto bias_c) {
+  auto stage_out = [&](auto silu_c, auto clamp_c, auto bias_c) {
     constexpr bool SILU = decltype(silu_c)::value;
     constexpr bool CLAMP = decltype(clamp_c)::value;
     constexpr bool HASB = decltype(bias_c)::value;
@@ -358,7 +360,8 @@ __global__ __launch_bounds__(512) void moe_gemm_wide_kernel(const GemmArgs a) {
       }
 #pragma unroll
       for (int j = 0; j < MG; ++j) {
-        const int srow = 32 * MG * wm + 32 * j + l32 - pass * PROWS;
+        if (j >= nj) break;  // uniform: the rows past them are the other half's or padding
+        const int srow = (PASSES == 1 ? rbase : 0) + 32 * j + l32;
         float ov[16];  // rounded to the 16-bit type once, in the packing below
 #pragma unroll
         for (int r = 0; r < 16; ++r) ov[r] = HASB ? acc[i][j][r] * es + bg[r] : acc[i][j][r] * es;
@@ -400,10 +403,10 @@ __global__ __launch_bounds__(512) void moe_gemm_wide_kernel(const GemmArgs a) {
   };
   using T_ = std::true_type;
   using F_ = std::false_type;
-  auto stage_pass = [&](int pass) {
+  auto stage_pass = [&]() {
     auto with_bias = [&](auto silu_c, auto clamp_c) {
-      if (a.bias) stage_out(pass, silu_c, clamp_c, T_{});
-      else stage_out(pass, silu_c, clamp_c, F_{});
+      if (a.bias) stage_out(silu_c, clamp_c, T_{});
+      else stage_out(silu_c, clamp_c, F_{});
     };
     if constexpr (!kGlu) {
       with_bias(T_{}, F_{});
@@ -420,11 +423,13 @@ __global__ __launch_bounds__(512) void moe_gemm_wide_kernel(const GemmArgs a) {
   };
 #pragma unroll
   for (int pass = 0; pass < PASSES; ++pass) {
-    if (PASSES == 1 || wm == pass) stage_pass(pass);
+    if (PASSES == 1 || wm == pass) stage_pass();
     __syncthreads();
-    for (int idx = tid; idx < PROWS * CPR; idx += 512) {
+    const int row0 = pass ? 32 * ng0 : 0;  // two passes: the rows of wave half `pass`
+    const int rows = (PASSES == 1 ? v : pass ? v - row0 : v < 32 * ng0 ? v : 32 * ng0);
+    for (int idx = tid; idx < rows * CPR; idx += 512) {
       const int srow = idx / CPR, ch = idx % CPR;
-      const int drow = s_drow[pass * PROWS + srow];
+      const int drow = s_drow[row0 + srow];
       const int64_t col = n0 + ch * 8;
       if (drow < 0 || col >= N) continue;
       const uint4 val = *reinterpret_cast<const uint4*>(lds + srow * PITCH + ch * 16);
