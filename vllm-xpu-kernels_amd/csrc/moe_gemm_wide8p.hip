@@ -1,6 +1,8 @@
 // Prefill grouped GEMM for fp8 e4m3 weights with 128x128 block scales and
 // e4m3 activations with 1x128 scales: 320-slot x 256-weight-row tiles, 8
-// waves, each wave owning 32 weight rows x all 320 slots.
+// waves in 2 x 4, each wave owning 64 weight rows x half of the block's valid
+// slot tiles (up to 160 slots).  With 32 weight rows x all 320 slots per wave
+// every wave read every activation row: 352 KB of LDS reads a stage, now 224.
 //
 // Data movement: both operands go global->LDS (global_load_lds), so no VGPR
 // holds data in flight.
@@ -10,24 +12,35 @@
 //     mostly L2 hits (every N-tile of an expert reads the same rows).  The
 //     transfer of stage kt + 1 is issued during stage kt, spread over the
 //     slot tiles.
-//   * weights (the HBM stream of the kernel): every wave moves its own two
-//     16-row fragments of a stage (4 KB) into its own region of a 2-slot
-//     weight ring, in lane order, two stages ahead: the transfer of stage
-//     kt + 2 goes out during stage kt after the activation parts, and the
-//     top of stage kt + 1 waits for all but those four newest transfers.  At
-//     the top of a stage each wave reads its fragments (four conflict-free
-//     16-byte LDS reads) into the operand registers, which frees the slot
-//     for the transfer two stages ahead.  Only the wave that wrote a weight
-//     region reads it, so the weights need no barrier.
-// Measured against loading the weights one stage ahead into VGPRs (C3,
-// T=8192): w2 1626 -> 1558 us, w13 2906 -> 2886 us per launch.
+//   * weights (the HBM stream of the kernel): every wave moves two of the
+//     sixteen 16-row fragments of a stage (4 KB) into a 2-slot weight ring,
+//     two stages ahead.  At the top of a stage each wave reads its four
+//     fragments (conflict-free 16-byte LDS reads) into the operand registers;
+//     a second barrier, before slot tile 6, says that all waves have, and the
+//     transfer of stage kt + 2 goes into the slot after it; the top of stage
+//     kt + 1 waits for all but those four newest transfers.  The second
+//     barrier costs nothing: it keeps the waves in step (without it, on data
+//     that is then wrong, w13 2266 -> 2361 us).
 //
-// Compute: per stage and wave 2 x 20 v_mfma_scale_f32_16x16x128_f8f6f4 (one
-// MFMA covers a whole 128-K scale block, unit e8m0 scales), each result
+// Compute: per stage and wave 4 x up to 10 v_mfma_scale_f32_16x16x128_f8f6f4
+// (one MFMA covers a whole 128-K scale block, unit e8m0 scales), each result
 // scaled and added with one FMA per element: acc += p * (xs * ws), the same
-// operations in the same order as the other fp8 kernels.  The 20 activation
-// fragments stream from LDS one tile ahead; slot tiles made only of padding
-// are skipped in pairs (the K loop is specialised on their number).
+// operations in the same order as the other fp8 kernels, two MFMAs after its
+// own.  The activation fragments stream from LDS one tile ahead; slot tiles
+// made only of padding are skipped (the K loop is specialised on the number
+// of tiles per half).  The order of MFMAs, FMAs and LDS reads is pinned with
+// sched_barrier: left to the compiler, reads were waited for right where they
+// were issued and FMAs right after their MFMA (w13 2266 -> 2240 us).
+//
+// What bounds it (DeepSeek-V3, 8192 tokens, w13, copies that leave parts
+// out): MFMAs and fixed cost alone 1462 us; without LDS fragment reads 1701,
+// without the DMA 1829, without the scaling FMAs 2041, whole 2266.  No one
+// path fills the time; the fixed cost (row ids, first transfers, epilogue,
+// with one workgroup on the CU) is 330 us of it.
+// Before / after the 2 x 4 split and the pinned order: w13 2353 -> 2240 us,
+// w2 1337 -> 1302 us; layers with a quarter of the intermediate size: fp8
+// 4096 tokens 960 -> 902, mxfp8 2048 / 8192 tokens 803 -> 731 / 1300 -> 1274;
+// gpt-oss-20b e2m1 x e2m1 1024 / 8192 tokens 192 -> 172 / 742 -> 732.
 //
 // LDS layout of an activation slot: rows of 128 bytes whose 16-byte chunk c
 // holds source chunk c ^ ((r >> 1) & 7), then the 320 scales in slot order
@@ -60,7 +73,7 @@ typedef __attribute__((address_space(1))) const i32x4_t gi32x4_t;
 constexpr int BM = 320, BN = 256, KE = 128;
 static_assert(BM == kWideBM, "block size of the WIDE family");
 constexpr int WAVES = 8;
-constexpr int TJ = BM / 16;                 // slot tiles per wave
+constexpr int TJ = BM / 32;                 // slot tiles per wave (half of the block's)
 constexpr int AROWS = BM / WAVES;           // activation rows moved per wave
 constexpr int A_BYTES = BM * KE;            // 40 KB of activations per stage
 constexpr int A_SLOT = A_BYTES + 2 * BM * 4;  // + scales (e2m1: two words of codes)
@@ -136,6 +149,7 @@ __global__ __launch_bounds__(512) void moe_gemm_wide8p_kernel(const GemmArgs a,
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, g = lane >> 4;
+  const int wn = wave & 3, wm = wave >> 2;  // weight quarter and slot half of the wave
 
   // XCD-aware order: XCD x takes the contiguous range [x*per, (x+1)*per) of
   // the tiles ordered by tile_coords (all N-tiles of an expert's block run
@@ -161,6 +175,10 @@ __global__ __launch_bounds__(512) void moe_gemm_wide8p_kernel(const GemmArgs a,
     s_arow[tid] = ok ? (a.a_by_pos ? blk * BM + tid : rid / a.a_div) : -1;
     s_drow[tid] = ok ? (a.d_by_pos ? blk * BM + tid : rid) : -1;
   }
+  // first tile row of weight fragment F
+  auto frag_row = [](int F) -> int {
+    return kGlu ? 32 * (F >> 2) + 16 * (F & 1) + ((F & 2) ? 128 : 0) : 16 * F;
+  };
   // weight row of tile row r (rows past N read row 0: finite data whose
   // outputs are never stored); GLU: [0,128) gate, [128,256) up
   auto wrow_of = [&](int r) -> int64_t {
@@ -226,10 +244,12 @@ __global__ __launch_bounds__(512) void moe_gemm_wide8p_kernel(const GemmArgs a,
   // byte step of the scale transfer from one K stage to the next
   // (MX by position: code word w of position P at (w * a_scale_tld + P) * 4)
   const uint32_t sstep = a.a_scale_tld ? static_cast<uint32_t>(a.a_scale_tld) * 4u : 4u;
-  // the wave's weight fragments f = 0, 1: GLU gate rows 16 wave + l16 and the
-  // matching up rows; STORE rows 32 wave + 16 f + l16.  Lane (l16, g) loads
-  // the 32 bytes at K byte 32 g of its row of the stage (mxfp8: the 16 bytes
-  // at 16 g and at 64 + 16 g, the scaled MFMA's e4m3 operand order).
+  // the stage's 16 weight fragments of 16 rows: fragments 4 c .. 4 c + 3 are
+  // the operands of the waves with wn = c, GLU gate rows 32 c + 16 f (f = 0,
+  // 1) and the matching up rows (f = 2, 3), STORE rows 64 c + 16 f; wave w
+  // moves fragments 2 w and 2 w + 1.  A lane (l16, g) uses the 32 bytes at K
+  // byte 32 g of its row of the stage (mxfp8: the 16 bytes at 16 g and at
+  // 64 + 16 g, the scaled MFMA's e4m3 operand order).
   // fp8 / mxfp8: a fragment's 16 rows x 128 bytes are staged like the
   // activation rows (LDS row t holds fragment row slot_of_lds_row(t), its
   // 16-byte chunk c source chunk c ^ swz(t)): transfer (f, h) moves LDS rows
@@ -243,7 +263,7 @@ __global__ __launch_bounds__(512) void moe_gemm_wide8p_kernel(const GemmArgs a,
     for (int h = 0; h < 2; ++h) {
       const int t = 8 * h + (lane >> 3);
       const int fr = slot_of_lds_row(t);
-      const int r = kGlu ? (f ? 128 : 0) + 16 * wave + fr : 32 * wave + 16 * f + fr;
+      const int r = frag_row(2 * wave + f) + fr;
       woff[f][h] = static_cast<uint32_t>(wrow_of(r) * wst.row) +
                    (static_cast<uint32_t>((lane & 7) ^ swz(t)) << 4);
     }
@@ -253,7 +273,7 @@ __global__ __launch_bounds__(512) void moe_gemm_wide8p_kernel(const GemmArgs a,
   if constexpr (MX4) {
 #pragma unroll
     for (int f = 0; f < 2; ++f) {
-      const int r = kGlu ? (f ? 128 : 0) + 16 * wave + l16 : 32 * wave + 16 * f + l16;
+      const int r = frag_row(2 * wave + f) + l16;
       woff[f][0] = static_cast<uint32_t>(wrow_of(r) * wst.row);
     }
   }
@@ -300,8 +320,8 @@ __global__ __launch_bounds__(512) void moe_gemm_wide8p_kernel(const GemmArgs a,
       dma4(soff + sstep * kt, sbase, s_wave ? slot + A_BYTES + 256 * wave : ring0 + DUMMY);
     }
   };
-  // weight fragments of stage kt: the wave's 4 KB region of weight slot
-  // `slot`, 1 KB per (fragment f, half h) in lane order
+  // weight fragments of stage kt: 2 KB each of weight slot `slot`, 1 KB per
+  // (fragment, half h) in lane order
   const uint32_t wring = ring0 + W_OFF + static_cast<uint32_t>(wave) * 4096u;
   auto issue_w = [&](int kt, int slot) {
     const uint32_t kofs = static_cast<uint32_t>(kt) * wkstep;
@@ -327,35 +347,28 @@ __global__ __launch_bounds__(512) void moe_gemm_wide8p_kernel(const GemmArgs a,
     dma4(coff + static_cast<uint32_t>(bc) * ldb, cbase,
          c_wave ? ring0 + C_OFF + slot * CSLOT + CPITCH * wave : ring0 + DUMMY);
   };
-  // the wave's weight fragments of ring slot `slot` (o0, o1: the activation
-  // fragment offsets of the lane)
-  auto read_w = [&](int slot, i32x8_t (&w)[2], int o0, int o1) {
-    if constexpr (MX4) {
-      const uint8_t* W = lds + W_OFF + slot * WSLOT + wave * 4096 + 16 * lane;
+  // the wave's weight fragments of ring slot `slot` (o0, o1: the fragment
+  // offsets of the lane)
+  auto read_w = [&](int slot, i32x8_t (&w)[4], int o0, int o1) {
+    const uint8_t* W = lds + W_OFF + slot * WSLOT + wn * 8192;
 #pragma unroll
-      for (int f = 0; f < 2; ++f) w[f] = ld32(W, 2 * f * 1024, (2 * f + 1) * 1024);
-    } else {
-      const uint8_t* W = lds + W_OFF + slot * WSLOT + wave * 4096;
-#pragma unroll
-      for (int f = 0; f < 2; ++f) w[f] = ld32(W + f * 2048, o0, o1);
-    }
+    for (int f = 0; f < 4; ++f)
+      w[f] = MX4 ? ld32(W + f * 2048 + 16 * lane, 0, 1024) : ld32(W + f * 2048, o0, o1);
   };
-  // tile rows of the lane's weight row l16 in fragments 0 and 1
-  const int rf0 = kGlu ? 16 * wave + l16 : 32 * wave + l16;
-  const int rf1 = kGlu ? 128 + 16 * wave + l16 : 32 * wave + 16 + l16;
   // mxfp8: e8m0 codes of the lane's weight rows for its 32-K block g
-  auto read_wc = [&](int slot, uint32_t (&c)[2]) {
+  auto read_wc = [&](int slot, uint32_t (&c)[4]) {
     const uint8_t* C = lds + C_OFF + slot * CSLOT + CPITCH * g;
-    c[0] = C[rf0];
-    c[1] = C[rf1];
+#pragma unroll
+    for (int f = 0; f < 4; ++f) c[f] = C[frag_row(4 * wn + f) + l16];
   };
   // e2m1: the same for blocks g (step 0) and 4 + g (step 1)
-  auto read_wc4 = [&](int slot, uint32_t (&c)[2][2]) {
+  auto read_wc4 = [&](int slot, uint32_t (&c)[4][2]) {
     const uint8_t* C = lds + C_OFF + slot * CSLOT + CPITCH * g;
-    c[0][0] = C[rf0];
-    c[0][1] = C[4 * CPITCH + rf0];
-    c[1][0] = C[rf1];
-    c[1][1] = C[4 * CPITCH + rf1];
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+      c[f][0] = C[frag_row(4 * wn + f) + l16];
+      c[f][1] = C[4 * CPITCH + frag_row(4 * wn + f) + l16];
+    }
   };
 
   // fragment offsets within an activation slot: chunks 2g and 2g + 1 of the
@@ -365,22 +378,22 @@ __global__ __launch_bounds__(512) void moe_gemm_wide8p_kernel(const GemmArgs a,
   const int xc0 = MX ? g : 2 * g, xc1 = MX ? g + 4 : 2 * g + 1;  // logical chunks
   const int xo0 = xr * KE + ((xc0 ^ swz(xr)) << 4);
   const int xo1 = xr * KE + ((xc1 ^ swz(xr)) << 4);
-  // s_wsc quarter of fragment f: GLU tile rows 16 wave (gate) and 128 +
-  // 16 wave (up); STORE rows 32 wave .. 32 wave + 31
-  const int wsel0 = kGlu ? (wave >> 2) : (wave >> 1), wsel1 = kGlu ? 2 + (wave >> 2) : (wave >> 1);
-  // slot tiles holding valid slots, rounded up to pairs
-  const int njv = (v + 15) / 16;
-  const int nj = njv <= 0 ? 0 : (njv >= TJ ? TJ : ((njv + 1) & ~1));
+  // s_wsc quarters of the wave: GLU gate (fragments 0, 1) and up (2, 3)
+  // rows, STORE rows 64 wn .. 64 wn + 63
+  const int wsel0 = kGlu ? wn >> 1 : wn, wsel1 = kGlu ? 2 + (wn >> 1) : wn;
+  // slot tiles per wave: the tiles holding valid slots, split evenly over
+  // the two slot halves; wave half wm computes tiles wm nj .. wm nj + nj - 1
+  const int nj = v <= 0 ? 0 : (v + 31) / 32;
 
-  f32x4_t acc[2][TJ];
+  f32x4_t acc[4][TJ];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < TJ; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   const int nk = nkb;
   // Stage kt: the six parts of the activation DMA of stage kt + 1 go out one
-  // every second slot tile (a wave that issues them back to back stalls
+  // every slot tile (a wave that issues them back to back stalls
   // until the DMA path takes them, and computes nothing meanwhile), then the
   // weight DMA of stage kt + 2; MX weight codes of stage kt + 1 go out first,
   // right after the barrier.  Transfers complete in issue order, so the wait
@@ -392,9 +405,17 @@ __global__ __launch_bounds__(512) void moe_gemm_wide8p_kernel(const GemmArgs a,
     constexpr int NJ = decltype(nj_c)::value;
     // slot tile after which part q of the activation DMA is issued (parts
     // past the last tile follow the loop)
-    auto part_at = [](int q) { return 2 * q; };
-    constexpr int W_AT = 11;   // tile after which the weight DMA of stage kt + 2 goes out
-    i32x8_t wc[2];
+    auto part_at = [](int q) { return q; };
+    constexpr int W_AT = 6;   // tile before which the weight DMA of stage kt + 2 goes out
+    // every wave holds its fragments of stage kt in registers: the weight
+    // slot of stage kt takes stage kt + 2
+    auto issue_w_next = [&](int kq, int slot) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      issue_w(kq, slot);
+    };
+    i32x8_t wc[4];
     if constexpr (MX) issue_c(0, 0);
 #pragma unroll
     for (int q = 0; q < ACT_PARTS; ++q) issue_act_part(q, 0, 0);
@@ -412,145 +433,132 @@ __global__ __launch_bounds__(512) void moe_gemm_wide8p_kernel(const GemmArgs a,
       // in stage kt - 1 (all are past the barrier); they land before the
       // weights issued later in this stage, so the wait above covers them
       if constexpr (MX) issue_c(kn, (kt + 1) & 1);
+      read_w(kt & 1, wc, xo0, xo1);
       if constexpr (MX4) {
         // last stage of a K % 256 != 0: zero this lane's weight chunks of
         // blocks past K (the DMA re-read the last block there; with a zero
         // weight operand the product is zero, e2m1 holding no Inf or NaN,
         // whatever the activation data and the finite codes)
         if (8 * kt + 8 > nblk) {
-          uint8_t* W = lds + W_OFF + (kt & 1) * WSLOT + wave * 4096 + 16 * lane;
 #pragma unroll
-          for (int f = 0; f < 2; ++f)
+          for (int h = 0; h < 2; ++h)
+            if (8 * kt + 4 * h + g >= nblk)
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
-              if (8 * kt + 4 * h + g >= nblk)
-                *reinterpret_cast<uint4*>(W + (2 * f + h) * 1024) = make_uint4(0, 0, 0, 0);
+              for (int f = 0; f < 4; ++f)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) wc[f][4 * h + k] = 0;
         }
       }
-      read_w(kt & 1, wc, xo0, xo1);
-      if constexpr (MX4 && NJ > 0) {
-        uint32_t wcode[2][2];
-        read_wc4(kt & 1, wcode);
-        const uint8_t* S = lds + (kt & 1) * A_SLOT;
-        const uint32_t* xsp = reinterpret_cast<const uint32_t*>(S + A_BYTES) + l16;
-        i32x8_t x = ld32(S, xo0, xo1);
-        // an e2m1 operand is four VGPRs: the low half of a fragment feeds
-        // K-step 0, the high half K-step 1.  Step 1 of tile j - 1 goes out
-        // with step 0 of tile j, so the two MFMAs into one accumulator are
-        // four apart, not two.
-        i32x8_t xp = x;
-        uint32_t xc1p = 0;
-        auto step1 = [&](int jj, const i32x8_t& xv, uint32_t xc) {
+      if constexpr (NJ > 0) {
+        uint32_t wcode[4][MX4 ? 2 : 1];
+        float ws0 = 0.f, ws1 = 0.f;
+        if constexpr (MX4) {
+          read_wc4(kt & 1, wcode);
+        } else if constexpr (MX) {
+          uint32_t c[4];
+          read_wc(kt & 1, c);
 #pragma unroll
-          for (int f = 0; f < 2; ++f)
-            acc[f][jj] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                __builtin_shufflevector(wc[f], wc[f], 4, 5, 6, 7, 0, 1, 2, 3),
-                __builtin_shufflevector(xv, xv, 4, 5, 6, 7, 0, 1, 2, 3), acc[f][jj], 4, 4, 0,
-                wcode[f][1], 0, xc);
+          for (int f = 0; f < 4; ++f) wcode[f][0] = c[f];
+        } else {
+          ws0 = s_wsc[wsel0][kt];
+          ws1 = s_wsc[wsel1][kt];
+        }
+        const uint8_t* S = lds + (kt & 1) * A_SLOT + wm * (NJ * 16 * KE);
+        const uint8_t* SC = lds + (kt & 1) * A_SLOT + A_BYTES + wm * (NJ * 64) + 4 * l16;
+        auto scale_of = [&](int j) { return *reinterpret_cast<const uint32_t*>(SC + 64 * j); };
+        auto scale2_of = [&](int j) {
+          return *reinterpret_cast<const uint32_t*>(SC + BM * 4 + 64 * j);
+        };
+        i32x8_t x = ld32(S, xo0, xo1);
+        uint32_t xs = scale_of(0), xs2 = MX4 ? scale2_of(0) : 0u;
+        // fp8: the scaling FMAs of a product follow two MFMAs later, so no
+        // wave waits for its own MFMA results
+        f32x4_t pq[2];
+        float s0 = 0.f, s1 = 0.f, t0 = 0.f, t1 = 0.f;  // of this tile, of the last one
+        auto scale_add = [&](int m, const f32x4_t& p, float a0, float a1) {
+          const float sc = (m & 3) < 2 ? a0 : a1;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[m & 3][m >> 2][r] += p[r] * sc;
         };
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
+          if (j == W_AT) issue_w_next(kq, kt & 1);
           i32x8_t xn = x;
-          if (j + 1 < NJ) xn = ld32(S + (j + 1) * 16 * KE, xo0, xo1);
-          const uint32_t xc0 = (xsp[16 * j] >> (8 * g)) & 0xffu;       // block g
-          const uint32_t xc1 = (xsp[BM + 16 * j] >> (8 * g)) & 0xffu;  // block 4 + g
-          if (j > 0) step1(j - 1, xp, xc1p);
+          uint32_t xsn = xs, xs2n = xs2;
+          if (j + 1 < NJ) {
+            xn = ld32(S + (j + 1) * 16 * KE, xo0, xo1);
+            xsn = scale_of(j + 1);
+            if constexpr (MX4) xs2n = scale2_of(j + 1);
+          }
+          if constexpr (MX4) {
+            // an e2m1 operand is four VGPRs: the low half of a fragment feeds
+            // K-step 0, the high half K-step 1, four MFMAs apart
+            const uint32_t xc0 = (xs >> (8 * g)) & 0xffu;   // block g
+            const uint32_t xc1 = (xs2 >> (8 * g)) & 0xffu;  // block 4 + g
 #pragma unroll
-          for (int f = 0; f < 2; ++f)
-            acc[f][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                wc[f], x, acc[f][j], 4, 4, 0, wcode[f][0], 0, xc0);
+            for (int f = 0; f < 4; ++f)
+              acc[f][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                  wc[f], x, acc[f][j], 4, 4, 0, wcode[f][0], 0, xc0);
 #pragma unroll
-          for (int q = 0; q < ACT_PARTS; ++q)
-            if (part_at(q) == j) issue_act_part(q, kn, kt + 1);
-          if (j == W_AT) issue_w(kq, kt & 1);
-          xp = x;
-          xc1p = xc1;
-          x = xn;
-        }
-        step1(NJ - 1, xp, xc1p);
-      } else if constexpr (MX && NJ > 0) {
-        uint32_t wcode[2];
-        read_wc(kt & 1, wcode);
-        const uint8_t* S = lds + (kt & 1) * A_SLOT;
-        const uint32_t* xsp = reinterpret_cast<const uint32_t*>(S + A_BYTES) + l16;
-        i32x8_t x = ld32(S, xo0, xo1);
+            for (int f = 0; f < 4; ++f)
+              acc[f][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                  __builtin_shufflevector(wc[f], wc[f], 4, 5, 6, 7, 0, 1, 2, 3),
+                  __builtin_shufflevector(x, x, 4, 5, 6, 7, 0, 1, 2, 3), acc[f][j], 4, 4, 0,
+                  wcode[f][MX4 ? 1 : 0], 0, xc1);
+          } else if constexpr (MX) {
+            const uint32_t xcode = (xs >> (8 * g)) & 0xffu;  // slot's 32-K block g
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          i32x8_t xn = x;
-          if (j + 1 < NJ) xn = ld32(S + (j + 1) * 16 * KE, xo0, xo1);
-          const uint32_t xcode = (xsp[16 * j] >> (8 * g)) & 0xffu;  // slot's 32-K block g
-          acc[0][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-              wc[0], x, acc[0][j], 0, 0, 0, wcode[0], 0, xcode);
-          acc[1][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-              wc[1], x, acc[1][j], 0, 0, 0, wcode[1], 0, xcode);
+            for (int f = 0; f < 4; ++f)
+              acc[f][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                  wc[f], x, acc[f][j], 0, 0, 0, wcode[f][0], 0, xcode);
+          } else {
+            t0 = s0;
+            t1 = s1;
+            s0 = __builtin_bit_cast(float, xs) * ws0;
+            s1 = kGlu ? __builtin_bit_cast(float, xs) * ws1 : s0;
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int q = 0; q < ACT_PARTS; ++q)
-            if (part_at(q) == j) issue_act_part(q, kn, kt + 1);
-          if (j == W_AT) issue_w(kq, kt & 1);
-          x = xn;
-        }
-      } else if constexpr (NJ > 0) {
-        const float ws0 = s_wsc[wsel0][kt], ws1 = s_wsc[wsel1][kt];
-        const uint8_t* S = lds + (kt & 1) * A_SLOT;
-        const float* xsp = reinterpret_cast<const float*>(S + A_BYTES) + l16;
-        // software pipeline: the scaling FMAs of slot tile j-1 follow the
-        // MFMAs of tile j, so no wave waits for its own MFMA results
-        i32x8_t x = ld32(S, xo0, xo1);
-        f32x4_t q0 = {0.f, 0.f, 0.f, 0.f}, q1 = q0;
-        float qs = 0.f;
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          i32x8_t xn = x;
-          if (j + 1 < NJ) xn = ld32(S + (j + 1) * 16 * KE, xo0, xo1);
-          const float xs = xsp[16 * j];
-          const f32x4_t p0 = mfma8(wc[0], x);
-          const f32x4_t p1 = mfma8(wc[1], x);
-#pragma unroll
-          for (int q = 0; q < ACT_PARTS; ++q)
-            if (part_at(q) == j) issue_act_part(q, kn, kt + 1);
-          if (j == W_AT) issue_w(kq, kt & 1);
-          if (j > 0) {
-            const float s0 = qs * ws0, s1 = qs * ws1;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              acc[0][j - 1][r] += q0[r] * s0;
-              acc[1][j - 1][r] += q1[r] * s1;
+            for (int f = 0; f < 4; ++f) {
+              const int m = 4 * j + f;
+              const f32x4_t p = mfma8(wc[f], x);
+              if (m >= 2) scale_add(m - 2, pq[m & 1], f < 2 ? t0 : s0, f < 2 ? t1 : s1);
+              pq[m & 1] = p;
+              __builtin_amdgcn_sched_barrier(0);
             }
           }
-          q0 = p0;
-          q1 = p1;
-          qs = xs;
-          x = xn;
-        }
-        {
-          const float s0 = qs * ws0, s1 = qs * ws1;
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            acc[0][NJ - 1][r] += q0[r] * s0;
-            acc[1][NJ - 1][r] += q1[r] * s1;
-          }
+          for (int q = 0; q < ACT_PARTS; ++q)
+            if (part_at(q) == j) issue_act_part(q, kn, kt + 1);
+          if constexpr (MX) __builtin_amdgcn_sched_barrier(0);
+          x = xn;
+          xs = xsn;
+          xs2 = xs2n;
+        }
+        if constexpr (!MX) {
+          scale_add(4 * NJ - 2, pq[0], s0, s1);
+          scale_add(4 * NJ - 1, pq[1], s0, s1);
         }
       }
 #pragma unroll
       for (int q = 0; q < ACT_PARTS; ++q)
         if (part_at(q) >= NJ) issue_act_part(q, kn, kt + 1);
-      if (NJ <= W_AT) issue_w(kq, kt & 1);
+      if (NJ <= W_AT) issue_w_next(kq, kt & 1);
     }
   };
   switch (nj) {
-    case 20: kloop(std::integral_constant<int, 20>{}); break;
-    case 18: kloop(std::integral_constant<int, 18>{}); break;
-    case 16: kloop(std::integral_constant<int, 16>{}); break;
-    case 14: kloop(std::integral_constant<int, 14>{}); break;
-    case 12: kloop(std::integral_constant<int, 12>{}); break;
     case 10: kloop(std::integral_constant<int, 10>{}); break;
+    case 9: kloop(std::integral_constant<int, 9>{}); break;
     case 8: kloop(std::integral_constant<int, 8>{}); break;
+    case 7: kloop(std::integral_constant<int, 7>{}); break;
     case 6: kloop(std::integral_constant<int, 6>{}); break;
+    case 5: kloop(std::integral_constant<int, 5>{}); break;
     case 4: kloop(std::integral_constant<int, 4>{}); break;
+    case 3: kloop(std::integral_constant<int, 3>{}); break;
     case 2: kloop(std::integral_constant<int, 2>{}); break;
+    case 1: kloop(std::integral_constant<int, 1>{}); break;
     default: kloop(std::integral_constant<int, 0>{}); break;
   }
-  static_assert(TJ == 20, "kloop variants cover the even tile counts up to TJ");
+  static_assert(TJ == 10, "kloop variants cover the tile counts up to TJ");
 
   // The epilogue, specialised on the activation, on gemm1_clamp_limit and on
   // the presence of a bias (uniform per launch), so that no value of the
@@ -559,17 +567,17 @@ __global__ __launch_bounds__(512) void moe_gemm_wide8p_kernel(const GemmArgs a,
     constexpr bool SILU = decltype(silu_c)::value;
     constexpr bool CLAMP = decltype(clamp_c)::value;
     constexpr bool HASB = decltype(bias_c)::value;
-    // ---- epilogue: lane holds slot 16 j + l16, rows 4 g + r of fragment f
+    // ---- epilogue: lane holds slot 16 (wm nj + j) + l16, rows 4 g + r of fragment f
     const int64_t bias_base = static_cast<int64_t>(e) * a.ldb_rows;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();  // the ring is free
     // output column (within the tile) of (fragment f, reg r)
     auto tcol = [&](int f, int r) -> int {
-      return (kGlu ? 16 * wave : 32 * wave + 16 * f) + 4 * g + r;
+      return (kGlu ? 32 * wn : 64 * wn) + 16 * f + 4 * g + r;
     };
-    constexpr int NF = kGlu ? 1 : 2;
+    constexpr int NF = kGlu ? 2 : 4;
     // the biases of the lane's output columns, the same for all its slots
-    float bgs[NF][4], bus[4];
+    float bgs[NF][4], bus[NF][4];
   #pragma unroll
     for (int f = 0; f < NF; ++f)
   #pragma unroll
@@ -577,7 +585,7 @@ __global__ __launch_bounds__(512) void moe_gemm_wide8p_kernel(const GemmArgs a,
         const int64_t n = n0 + tcol(f, r);
         const bool has = HASB && n < N;
         bgs[f][r] = has ? ld16<F16>(a.bias[bias_base + n]) : 0.f;
-        if (f == 0) bus[r] = has && kGlu ? ld16<F16>(a.bias[bias_base + a.up_off + n]) : 0.f;
+        bus[f][r] = has && kGlu ? ld16<F16>(a.bias[bias_base + a.up_off + n]) : 0.f;
       }
     // the lane's four outputs of (fragment f, slot tile j) before their final
     // rounding to the 16-bit type: GLU act(round16(gate), round16(up)),
@@ -589,7 +597,8 @@ __global__ __launch_bounds__(512) void moe_gemm_wide8p_kernel(const GemmArgs a,
       if constexpr (kGlu) {
         float u[4];
   #pragma unroll
-        for (int r = 0; r < 4; ++r) u[r] = HASB ? acc[1][j][r] + bus[r] : acc[1][j][r];
+        for (int r = 0; r < 4; ++r)
+          u[r] = HASB ? acc[f + 2][j][r] + bus[f][r] : acc[f + 2][j][r];
         round16xn<F16>(gv);
         round16xn<F16>(u);
         if constexpr (CLAMP)
@@ -627,17 +636,21 @@ __global__ __launch_bounds__(512) void moe_gemm_wide8p_kernel(const GemmArgs a,
       constexpr int P16 = 2 * NOUT + 16;  // staging row pitch (bytes)
   #pragma unroll
       for (int j = 0; j < TJ; ++j) {
-        float o[4];
-        outv(0, j, o);
-        *reinterpret_cast<uint2*>(lds + (16 * j + l16) * P16 + 2 * tcol(0, 0)) =
-            make_uint2(pack16x2<F16>(o[0], o[1]), pack16x2<F16>(o[2], o[3]));
+        if (j >= nj) break;
+  #pragma unroll
+        for (int f = 0; f < NF; ++f) {
+          float o[4];
+          outv(f, j, o);
+          *reinterpret_cast<uint2*>(lds + (16 * (wm * nj + j) + l16) * P16 + 2 * tcol(f, 0)) =
+              make_uint2(pack16x2<F16>(o[0], o[1]), pack16x2<F16>(o[2], o[3]));
+        }
       }
       __syncthreads();
       float* ds = static_cast<float*>(qs);
       uint8_t* dq = static_cast<uint8_t*>(a.D);
       const int64_t ngroups = N / 128;
       const int c = tid & 15;  // the lane's 8-column chunk of the row
-      for (int row = tid >> 4; row < BM; row += 512 / 16) {  // every lane, every pass
+      for (int row = tid >> 4; row < 32 * nj; row += 512 / 16) {  // every lane, every pass
         const uint4 u = *reinterpret_cast<const uint4*>(lds + row * P16 + 16 * c);
         float x[8];
         unpack16x2<F16>(u.x, x[0], x[1]);
@@ -673,10 +686,14 @@ __global__ __launch_bounds__(512) void moe_gemm_wide8p_kernel(const GemmArgs a,
       constexpr int P16 = 2 * NOUT + 16;  // staging row pitch (bytes)
   #pragma unroll
       for (int j = 0; j < TJ; ++j) {
-        float o[4];
-        outv(0, j, o);
-        *reinterpret_cast<uint2*>(lds + (16 * j + l16) * P16 + 2 * tcol(0, 0)) =
-            make_uint2(pack16x2<F16>(o[0], o[1]), pack16x2<F16>(o[2], o[3]));
+        if (j >= nj) break;
+  #pragma unroll
+        for (int f = 0; f < NF; ++f) {
+          float o[4];
+          outv(f, j, o);
+          *reinterpret_cast<uint2*>(lds + (16 * (wm * nj + j) + l16) * P16 + 2 * tcol(f, 0)) =
+              make_uint2(pack16x2<F16>(o[0], o[1]), pack16x2<F16>(o[2], o[3]));
+        }
       }
       __syncthreads();
       uint8_t* dq = static_cast<uint8_t*>(a.D);
@@ -684,7 +701,7 @@ __global__ __launch_bounds__(512) void moe_gemm_wide8p_kernel(const GemmArgs a,
       const int64_t orow = MX4 ? (a.ldd ? a.ldd : N / 2) : N;  // output row pitch (bytes)
       const int c = tid & 15;  // the lane's 8-column chunk of the row
       const int p = c >> 2;    // its 32-column group
-      for (int row = tid >> 4; row < BM; row += 512 / 16) {  // every lane, every pass
+      for (int row = tid >> 4; row < 32 * nj; row += 512 / 16) {  // every lane, every pass
         const uint4 u = *reinterpret_cast<const uint4*>(lds + row * P16 + 16 * c);
         float x[8];
         unpack16x2<F16>(u.x, x[0], x[1]);
@@ -728,9 +745,9 @@ __global__ __launch_bounds__(512) void moe_gemm_wide8p_kernel(const GemmArgs a,
       // 16-bit output staged in LDS (STORE tiles in two passes of 160 slots)
       // and written with 16-byte row-contiguous stores
       constexpr int PITCH = 2 * NOUT + 16;
-      // passes of a whole number of slot tiles each, as few as the ring holds
-      constexpr int PASSES = BM * PITCH <= RING ? 1 : BM / 2 * PITCH <= RING ? 2
-                           : BM / 4 * PITCH <= RING ? 4 : 5;
+      // passes of the same slot tiles of both wave halves, as few as the ring
+      // holds: tile jj of half h is staged at rows 16 (PJ h + jj)
+      constexpr int PASSES = BM * PITCH <= RING ? 1 : 2;
       static_assert(BM / PASSES * PITCH <= RING && TJ % PASSES == 0, "staging passes");
       constexpr int PROWS = BM / PASSES;
       constexpr int PJ = TJ / PASSES;
@@ -744,9 +761,10 @@ __global__ __launch_bounds__(512) void moe_gemm_wide8p_kernel(const GemmArgs a,
   #pragma unroll
           for (int jj = 0; jj < PJ; ++jj) {
             const int j = pass * PJ + jj;
+            if (j >= nj) break;
             float o[4];
             outv(f, j, o);
-            const int srow = 16 * jj + l16;
+            const int srow = 16 * (wm * PJ + jj) + l16;
             const uint32_t lo = pack16x2<F16>(o[0], o[1]);
             const uint32_t hi = pack16x2<F16>(o[2], o[3]);
             *reinterpret_cast<uint2*>(lds + srow * PITCH + 2 * tcol(f, 0)) = make_uint2(lo, hi);
@@ -754,9 +772,12 @@ __global__ __launch_bounds__(512) void moe_gemm_wide8p_kernel(const GemmArgs a,
         __syncthreads();
         for (int idx = tid; idx < PROWS * CPR; idx += 512) {
           const int srow = idx / CPR, ch = idx % CPR;
-          const int drow = s_drow[pass * PROWS + srow];
+          const int h = srow >= 16 * PJ;  // wave half and its slot tile
+          const int j = pass * PJ + (srow >> 4) - PJ * h;
           const int64_t col = n0 + ch * 8;
-          if (drow < 0 || col >= N) continue;
+          if (j >= nj || col >= N) continue;
+          const int drow = s_drow[16 * (h * nj + j) + (srow & 15)];
+          if (drow < 0) continue;
           const uint4 val = *reinterpret_cast<const uint4*>(lds + srow * PITCH + ch * 16);
           uint16_t* dst = d + static_cast<int64_t>(drow) * N + col;
           if (vec) {
