@@ -69,3 +69,30 @@ def test_layer_tiles_per_half(dev, recipe):
         moe.apply(out, x.to(dev), tw.to(dev), ti.to(dev))
     ref = O.fused_moe(recipe, x, *ora, tw, ti, a1q_scale=xs)
     _close_fp8(out.cpu(), ref)
+
+
+def test_layer_in_short_scratch(dev):
+    """56 slots per expert: 320-slot blocks pad the activation beyond the
+    static 64 MiB scratch of the allocation-free entry, which then runs
+    64-slot blocks; both against each other to the fp8 layer bar."""
+    import ctypes
+    import dataclasses
+
+    from vllm_xpu_kernels import capi
+    from vllm_xpu_kernels import workloads as W
+    cfg, T = dataclasses.replace(W.config("C2"), recipe="fp8block"), 900
+    print(f"wide8p short scratch: {cfg.name} {cfg.recipe} T={T}", flush=True)
+    w = W.make_weights(cfg, dev)
+    moe = _layer_cls()(*w.layer_args(), cfg.topk, cfg.activation, cfg.experts)
+    x = W.make_activations(cfg, T, dev, seed=3)
+    tw, ti = W.route(cfg, W.make_router_logits(cfg, T, dev, seed=4), None)
+    ref, out = torch.empty_like(x), torch.full_like(x, float("nan"))
+    moe.apply(ref, x, tw, ti)
+    a = capi.fused_args(moe, out, x, tw, ti)
+    assert capi.workspace_for(a, dev).numel() > 64 << 20
+    capi.lib.mi355moe_fused_moe_noalloc.argtypes = [ctypes.POINTER(capi.FusedMoeArgs),
+                                                    ctypes.c_void_p]
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    rc = capi.lib.mi355moe_fused_moe_noalloc(ctypes.byref(a), stream)
+    assert rc == 0, capi.lib.mi355moe_last_error()
+    _close_fp8(out.cpu(), ref.cpu())

@@ -534,7 +534,8 @@ bool stream_khalves_enabled() {
   return !(v && v[0] == '0');
 }
 
-// max_bm: SMALL blocks of at most that many slots (plan() below)
+// max_bm: blocks of at most that many slots where SMALL can take them
+// (plan() below); kWideBM: the preferred family
 FusedLayout plan_with(const mi355moe_fused_moe_args* a, uint8_t* base, int max_bm) {
   FusedLayout L{};
   const int64_t E = a->num_experts;
@@ -550,6 +551,7 @@ FusedLayout plan_with(const mi355moe_fused_moe_args* a, uint8_t* base, int max_b
   int64_t local = L.slots;
   if (a->expert_map && a->expert_map_len > E) local = cdiv(L.slots * E, a->expert_map_len);
   L.tile = pick_tile(gemm_recipe(a), wide_ok, L.slots, local, E, &L.bm);
+  if (L.tile == TILE_WIDE && max_bm < kWideBM) L.tile = TILE_SMALL;
   if (L.tile == TILE_SMALL && !(mid_fits(2 * I, H) && mid_fits(H, K2))) {
     L.tile = TILE_STREAM;  // 64-bit weight offsets
     L.bm = 16;
@@ -641,9 +643,13 @@ FusedLayout plan_with(const mi355moe_fused_moe_args* a, uint8_t* base, int max_b
 }
 
 // The layer's plan in a workspace of `limit` bytes: where the preferred SMALL
-// blocks pad the activation beyond it, smaller ones.
+// blocks, or the 320-slot blocks of fp8 block-scaled weights up to 160 slots
+// per expert, pad the activation beyond it, smaller SMALL blocks.
 FusedLayout plan(const mi355moe_fused_moe_args* a, uint8_t* base, size_t limit = SIZE_MAX) {
-  FusedLayout L = plan_with(a, base, 128);
+  FusedLayout L = plan_with(a, base, kWideBM);
+  if (L.bytes > limit && L.tile == TILE_WIDE && gemm_recipe(a) == MI355MOE_RECIPE_FP8BLOCK &&
+      L.slots <= 160 * std::min<int64_t>(L.slots, a->num_experts))
+    L = plan_with(a, base, 64);
   while (L.bytes > limit && L.tile == TILE_SMALL && L.bm > 16)
     L = plan_with(a, base, L.bm > 64 ? 64 : L.bm / 2);
   return L;
