@@ -17,8 +17,10 @@ namespace {
 //                     37: 351 302 251 255 262      56: 435 323 276 262 268 W 291
 //                     87: 584 380 332 305 286 W 304   125: - - 384 385 367 W 325
 //   fp8   rank of 8 of DeepSeek-V3  4: 246 245 258 269 -   12: 319 271 282 290 -
-//                     31: 549 411 301 310 - W 333  44: 617 430 315 321 - W 342
-//         DeepSeek-V3 whole         56: - - 2479 2319 - W 2351   64: - - 2760 2423 - W 2388
+//                     31: 549 411 301 310 -   40: - - 316 - - W 320
+//                     52: - - - 341 - W 332  58: - - - 352 - W 340
+//         DeepSeek-V3 whole         40: - - 2164 - - W 2134   47: - - - 2242 - W 2174
+//                                   58: - - 2479 2364 - W 2244
 //   w8a16 rank of 8 of DeepSeek-V3  3: 241 244 249 270 -   16: 355 281 282 304 -
 //                     32: 525 382 297 302 324 W 365   62: - - 421 376 386 W 437
 //                     94: - - 467 476 498 W 509
@@ -28,9 +30,10 @@ namespace {
 //   mxfp4 gpt-oss-20b 8: 100 105 120 - -   16: 121 109 124 145 196
 //                     25: 130 123 129 148 199   37: 182 153 144 160 212
 //                     65: 256 207 217 188 245 W 306   112: - 285 278 320 297 W 342
-int small_block(int recipe, int64_t avg) {
+int small_block(int recipe, int64_t avg, bool wide_ok) {
   if (recipe == MI355MOE_RECIPE_FP8BLOCK)
-    return avg <= 4 ? 16 : avg <= 18 ? 32 : avg <= 46 ? 64 : avg <= 60 ? 96 : 0;
+    return avg <= 4 ? 16 : avg <= 18 ? 32 : avg <= (wide_ok ? 44 : 46) ? 64
+           : avg <= 60 && !wide_ok ? 96 : 0;
   if (is_w8a16_recipe(recipe))
     return avg <= 4 ? 16 : avg <= 17 ? 32 : avg <= 46 ? 64 : avg <= 100 ? 96 : 0;
   if (recipe == MI355MOE_RECIPE_INT4)
@@ -69,7 +72,7 @@ GemmTile pick_tile(int recipe, bool wide_ok, int64_t slots, int64_t local, int64
   }();
   const int64_t active = local < num_experts ? local : num_experts;
   const int64_t avg = active > 0 ? local / active : 0;
-  const int sb = small_block(recipe, avg);
+  const int sb = small_block(recipe, avg, wide_ok);
   GemmTile t;
   int b;
   if ((recipe == MI355MOE_RECIPE_MXFP8 || recipe == RECIPE_MX4A4) && wide_ok && avg > 16) {
