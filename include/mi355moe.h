@@ -515,11 +515,13 @@ int mi355moe_fused_moe(const mi355moe_fused_moe_args* args, void* workspace,
  * reference: it is for callers that cannot allocate (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  The
  * workspace is a static device array of MI355MOE_NOALLOC_SCRATCH_BYTES per GPU
- * (held until the process ends); the call allocates nothing and returns
- * MI355MOE_ERR_WORKSPACE when mi355moe_fused_moe_workspace_size(args) exceeds
- * it (64 MiB covers decode batches: DeepSeek-V3 shape up to 256 tokens,
- * Qwen3-30B-A3B up to 512).  Calls that overlap on one GPU share that array
- * and race. */
+ * (held until the process ends); the call allocates nothing.  Where
+ * mi355moe_fused_moe_workspace_size(args) exceeds it, the layer pads to smaller
+ * blocks of slots if those fit, which takes longer and whose result may differ
+ * from mi355moe_fused_moe's in rounding; where even those do not fit it returns
+ * MI355MOE_ERR_WORKSPACE.  64 MiB covers decode batches: DeepSeek-V3 shape up
+ * to 361 tokens (424 with smaller blocks), Qwen3-30B-A3B up to 1072 (1421).
+ * Calls that overlap on one GPU share that array and race. */
 #define MI355MOE_NOALLOC_SCRATCH_BYTES ((size_t)64 << 20)
 int mi355moe_fused_moe_noalloc(const mi355moe_fused_moe_args* args, void* stream);
 

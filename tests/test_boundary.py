@@ -443,6 +443,27 @@ def test_fused_moe_noalloc_rejects_calls_beyond_its_scratch(lib):
     assert b"more than the static" in lib.mi355moe_last_error()
 
 
+@pytest.mark.parametrize("name,kw", [
+    # plans with 320-slot fp8 blocks, and SMALL blocks of 32 to 128 slots
+    ("fp8 wide", dict(recipe=1, num_tokens=900, hidden=2048, inter=768, num_experts=128)),
+    ("fp8 small", dict(recipe=1, num_tokens=400, hidden=7168, inter=2048, num_experts=256)),
+    ("int4", dict(recipe=3, num_tokens=300, hidden=2048, inter=768, num_experts=128,
+                  w_group=128)),
+    ("bf16", dict(recipe=0, num_tokens=1500, hidden=2048, inter=768, num_experts=128)),
+    ("mxfp4", dict(recipe=2, num_tokens=400, hidden=2880, inter=2880, num_experts=32))])
+def test_fused_moe_refuses_short_workspace(lib, name, kw):
+    """The caller-workspace entry refuses, before any device work, a workspace
+    below mi355moe_fused_moe_workspace_size, also by one byte and where
+    smaller blocks of slots would fit it."""
+    from vllm_xpu_kernels import capi
+    a = capi.FusedMoeArgs(activation=0, act_dtype=1, ids_dtype=3, topk=8, w_layout=1,
+                          w13_scale=1, w2_scale=1, **kw)
+    need = lib.mi355moe_fused_moe_workspace_size(ctypes.byref(a))
+    for short in (need - 1, need - 4096, need * 3 // 4, need // 2):
+        rc = lib.mi355moe_fused_moe(ctypes.byref(a), ctypes.c_void_p(256), short, None)
+        assert rc == -4 and b"workspace too small" in lib.mi355moe_last_error(), (name, short)
+
+
 @pytest.mark.parametrize("field,value,message", [
     ("num_tokens", -1, b"invalid layer shape"), ("topk", 0, b"invalid layer shape"),
     ("num_experts", 2048, b"at most 1024"), ("hidden", 7100, b"% 128"),

@@ -535,7 +535,7 @@ bool stream_khalves_enabled() {
 }
 
 // max_bm: blocks of at most that many slots where SMALL can take them
-// (plan() below); kWideBM: the preferred family
+// (plan_within() below); kWideBM: the preferred family
 FusedLayout plan_with(const mi355moe_fused_moe_args* a, uint8_t* base, int max_bm) {
   FusedLayout L{};
   const int64_t E = a->num_experts;
@@ -642,11 +642,19 @@ FusedLayout plan_with(const mi355moe_fused_moe_args* a, uint8_t* base, int max_b
   return L;
 }
 
-// The layer's plan in a workspace of `limit` bytes: where the preferred SMALL
-// blocks, or the 320-slot blocks of fp8 block-scaled weights up to 160 slots
-// per expert, pad the activation beyond it, smaller SMALL blocks.
-FusedLayout plan(const mi355moe_fused_moe_args* a, uint8_t* base, size_t limit = SIZE_MAX) {
-  FusedLayout L = plan_with(a, base, kWideBM);
+// The layer's plan in a caller's workspace: a function of the arguments alone.
+FusedLayout plan(const mi355moe_fused_moe_args* a, uint8_t* base) {
+  return plan_with(a, base, kWideBM);
+}
+
+// The plan of the allocation-free entry, whose scratch has a fixed size: where
+// the preferred SMALL blocks, or the 320-slot blocks of fp8 block-scaled
+// weights up to 160 slots per expert, pad the activation beyond `limit` bytes,
+// smaller SMALL blocks.  Their results can differ from the preferred plan's in
+// rounding: the 320-slot kernel's activation function is another than SMALL's,
+// and 16-slot int4 blocks scale sums instead of weights.
+FusedLayout plan_within(const mi355moe_fused_moe_args* a, uint8_t* base, size_t limit) {
+  FusedLayout L = plan(a, base);
   if (L.bytes > limit && L.tile == TILE_WIDE && gemm_recipe(a) == MI355MOE_RECIPE_FP8BLOCK &&
       L.slots <= 160 * std::min<int64_t>(L.slots, a->num_experts))
     L = plan_with(a, base, 64);
@@ -669,7 +677,7 @@ namespace mi355 {
 namespace {
 int validate(const mi355moe_fused_moe_args* a);
 int fused_moe_impl(const mi355moe_fused_moe_args* a, void* ws, size_t ws_bytes,
-                   void* stream, hipEvent_t* ev);
+                   void* stream, hipEvent_t* ev, bool fixed_scratch = false);
 }
 }  // namespace mi355
 
@@ -723,7 +731,7 @@ int scratch_address(hipStream_t stream, void** out) {
 
 extern "C" int mi355moe_fused_moe_noalloc(const mi355moe_fused_moe_args* a, void* stream) {
   if (int rc = validate(a)) return rc;   // before the arguments size anything
-  const size_t need = plan(a, nullptr, MI355MOE_NOALLOC_SCRATCH_BYTES).bytes;
+  const size_t need = plan_within(a, nullptr, MI355MOE_NOALLOC_SCRATCH_BYTES).bytes;
   MI_CHECK(need <= MI355MOE_NOALLOC_SCRATCH_BYTES, MI355MOE_ERR_WORKSPACE,
            "fused_moe_noalloc: this call needs " + std::to_string(need) +
                " bytes of scratch, more than the static " +
@@ -731,7 +739,8 @@ extern "C" int mi355moe_fused_moe_noalloc(const mi355moe_fused_moe_args* a, void
                " (use mi355moe_fused_moe with a caller workspace)");
   void* ptr = nullptr;
   if (int rc = scratch_address(static_cast<hipStream_t>(stream), &ptr)) return rc;
-  return fused_moe_impl(a, ptr, MI355MOE_NOALLOC_SCRATCH_BYTES, stream, nullptr);
+  return fused_moe_impl(a, ptr, MI355MOE_NOALLOC_SCRATCH_BYTES, stream, nullptr,
+                        /*fixed_scratch=*/true);
 }
 
 extern "C" int mi355moe_timer_create(int max_steps, mi355moe_timer* out) {
@@ -838,15 +847,17 @@ int validate(const mi355moe_fused_moe_args* a) {
   return MI355MOE_OK;
 }
 
+// fixed_scratch: the allocation-free entry's workspace (plan_within)
 int fused_moe_impl(const mi355moe_fused_moe_args* a, void* ws, size_t ws_bytes,
-                   void* stream, hipEvent_t* ev) {
+                   void* stream, hipEvent_t* ev, bool fixed_scratch) {
   if (int rc = validate(a)) return rc;
   const int64_t T = a->num_tokens, H = a->hidden, I = a->inter, E = a->num_experts,
                 k = a->topk;
   const int recipe = a->recipe;
   const bool kblock = a->w_layout == MI355MOE_WLAYOUT_KBLOCK;
   if (T == 0) return MI355MOE_OK;
-  FusedLayout L = plan(a, static_cast<uint8_t*>(ws), ws_bytes);
+  uint8_t* base = static_cast<uint8_t*>(ws);
+  FusedLayout L = fixed_scratch ? plan_within(a, base, ws_bytes) : plan(a, base);
   MI_CHECK(ws && ws_bytes >= L.bytes, MI355MOE_ERR_WORKSPACE,
            "workspace too small for fused_moe");
   hipStream_t st = static_cast<hipStream_t>(stream);
