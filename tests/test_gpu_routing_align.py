@@ -233,6 +233,24 @@ def test_moe_align_block_size_bit_exact(dev, m, topk, E, bs, id_dtype):
     assert np.array_equal(srt.cpu().numpy(), rs)
 
 
+@pytest.mark.parametrize("m", [40, 4100])
+@pytest.mark.parametrize("E", [1, 16, 17, 512, 513, 990])
+@pytest.mark.parametrize("bs", [1, 16, 320])
+def test_moe_align_padding_lanes(dev, m, E, bs):
+    """The padding of an expert is written by the 64 down to 1 lanes that the
+    launch has per expert: on both sides of the powers of two, with most
+    experts empty (few distinct ids) and with blocks wider than their lanes."""
+    g = torch.Generator().manual_seed(m + E)
+    ids = torch.randint(0, E, (m, 1), generator=g, dtype=torch.int32)
+    ids[::2] = E - 1
+    srt, eids, ntp = _ops().moe_align_block_size(ids.to(dev), bs, E)
+    mx, nb = O.align_buffer_sizes(ids.numel(), E, bs)
+    rs, re, rn = O.moe_align_block_size(ids, E, bs, mx, nb)
+    assert ntp.cpu().tolist() == rn.tolist()
+    assert np.array_equal(eids.cpu().numpy(), re)
+    assert np.array_equal(srt.cpu().numpy(), rs)
+
+
 def test_moe_align_zipf_skew_c4(dev):
     from vllm_xpu_kernels import workloads as W
     cfg = W.CONFIGS["C4"]
