@@ -97,6 +97,15 @@ __device__ int block_exclusive_scan(int v, int* s_wave_tot, int& total) {
 // Bits that tell the keys 0 .. num_keys - 1 and kInvalidKey (all ones) apart.
 __device__ __forceinline__ int key_bits(int num_keys) { return 32 - __clz(num_keys); }
 
+// LDS that the lanes of one wave exchange: no access may cross it.  The
+// hardware executes a wave's LDS accesses in program order, so it costs no
+// instruction; without it the compiler may sink one lane's read below another
+// lane's write.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
 // Output slot of this lane's key: the wave's next slot of that key (cnt,
 // advanced past the wave's ids of it) plus the lanes below with the same key;
 // -1 for kInvalidKey.  All 64 lanes must be active.
@@ -107,11 +116,11 @@ __device__ __forceinline__ int place(uint32_t key, int bits, int lane, int* cnt)
     same &= ((key >> b) & 1u) ? bb : ~bb;
   }
   const int rank = __popcll(same & ((1ull << lane) - 1ull));
-  int pos = -1;
-  if (key != kInvalidKey) {
-    pos = cnt[key] + rank;
-    if (rank == 0) cnt[key] += __popcll(same);
-  }
+  const bool ok = key != kInvalidKey;
+  const int pos = ok ? cnt[key] + rank : -1;
+  wave_lds_order();  // every lane has read the counter that the first lane of its key moves
+  if (ok && rank == 0) cnt[key] = pos + __popcll(same);
+  wave_lds_order();  // read by the next step's lanes
   return pos;
 }
 
@@ -256,8 +265,7 @@ __device__ __forceinline__ void counting_sort_body(
   }
   __syncthreads();
 
-  // phase 3: stable scatter (a wave's counters are its own, and the LDS
-  // accesses of one wave execute in program order)
+  // phase 3: stable scatter (a wave's counters are its own)
   const int bits = key_bits(num_keys);
   auto step = [&](int s, uint32_t key) {
     const int64_t i = lo + static_cast<int64_t>(s) * 64 + lane;
