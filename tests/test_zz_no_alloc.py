@@ -70,3 +70,28 @@ def test_fused_moe_noalloc_expert_map(dev):
     assert moe.expert_map is not None and moe.expert_map.numel() == 32
     for i, T in enumerate((33, 2)):
         _run_pair(cfg, T, dev, moe, w, seed=40 + 3 * i, expert_map=moe.expert_map)
+
+
+@pytest.mark.parametrize("T", [2, 60, 700])
+def test_fused_moe_empty_expert_map(dev, T):
+    """A C caller's map of no entries (the pointer's one word is beyond it):
+    every id lies outside it and the output is zero, in the streaming, SMALL
+    and prefill families."""
+    from vllm_xpu_kernels import capi
+    from vllm_xpu_kernels import workloads as W
+    from vllm_xpu_kernels.fused_moe_interface import XpuFusedMoe
+    cfg = W.config("C1")
+    w = W.make_weights(cfg, dev)
+    moe = XpuFusedMoe(*w.layer_args(), cfg.topk, cfg.activation, cfg.experts)
+    x = W.make_activations(cfg, T, dev, seed=2)
+    tw, ti = W.route(cfg, W.make_router_logits(cfg, T, dev, seed=3), None)
+    out = torch.full_like(x, float("nan"))
+    entry = torch.zeros(1, dtype=torch.int32, device=dev)
+    a = capi.fused_args(moe, out, x, tw, ti, expert_map=entry)
+    a.expert_map_len = 0
+    ws = capi.workspace_for(a, dev)
+    rc = capi.lib.mi355moe_fused_moe(ctypes.byref(a), ctypes.c_void_p(ws.data_ptr()),
+                                     ctypes.c_size_t(ws.numel()),
+                                     ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0, capi.lib.mi355moe_last_error()
+    assert torch.equal(out, torch.zeros_like(out))

@@ -56,7 +56,8 @@ int64_t launch_blocks(int64_t slots, int64_t experts, int64_t bm,
 // the sort kept, in j order.  MAP (expert parallelism): most slots are other
 // ranks' -- their ids and map entries are read together first, and a dropped
 // slot moves no bytes (a rank of 8, 1003 tokens of 7168: 15.4 -> 9 us); without
-// a map every slot is in and its row is requested at once.
+// a map every slot is in and its row is requested at once.  MAP needs
+// map_len > 0: ids outside the map read its first entry.
 template <typename Id, bool F16, bool MAP>
 __global__ __launch_bounds__(256) void weighted_topk_sum_kernel(
     uint16_t* __restrict__ out, const uint16_t* __restrict__ g2,
@@ -1160,15 +1161,18 @@ int fused_moe_impl(const mi355moe_fused_moe_args* a, void* ws, size_t ws_bytes,
   // Slots dropped by the sort (invalid or non-local experts) were never
   // written by the w2 GEMM; the reduction skips them by the same rule.
   dim3 grid(static_cast<unsigned>(cdiv(cdiv(H, 8), 256)), static_cast<unsigned>(T));
+  // an empty map has no entry to read and routes no slot here
+  const bool mapped = a->expert_map && a->expert_map_len > 0;
+  const int64_t experts = a->expert_map && !mapped ? 0 : E;
   auto reduce = [&](auto id_tag, auto f16_tag, auto map_tag) {
     using Id = decltype(id_tag);
     weighted_topk_sum_kernel<Id, decltype(f16_tag)::value, decltype(map_tag)::value>
         <<<grid, dim3(256), 0, st>>>(static_cast<uint16_t*>(a->output), L.g2, a->topk_weights,
                                      static_cast<const Id*>(a->topk_ids), a->expert_map,
-                                     a->expert_map_len, E, T, static_cast<int>(k), H);
+                                     a->expert_map_len, experts, T, static_cast<int>(k), H);
   };
   auto with_map = [&](auto id_tag, auto f16_tag) {
-    if (a->expert_map) reduce(id_tag, f16_tag, std::true_type{});
+    if (mapped) reduce(id_tag, f16_tag, std::true_type{});
     else reduce(id_tag, f16_tag, std::false_type{});
   };
   auto with_type = [&](auto id_tag) {
