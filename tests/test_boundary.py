@@ -464,6 +464,26 @@ def test_fused_moe_refuses_short_workspace(lib, name, kw):
         assert rc == -4 and b"workspace too small" in lib.mi355moe_last_error(), (name, short)
 
 
+@pytest.mark.parametrize("recipe,hidden,inter", [
+    # 2^31 weights per w13 expert and more: neither the 320-slot kernel's nor
+    # SMALL's 32-bit offsets (bf16; int4, whose offsets are a quarter of it)
+    (0, 32768, 32768), (3, 65536, 65536)])
+@pytest.mark.parametrize("tokens", [40, 300, 5000])
+def test_fused_moe_huge_experts_stream(lib, monkeypatch, recipe, hidden, inter, tokens):
+    """K-blocked experts beyond the 32-bit offsets of the SMALL and WIDE
+    kernels plan the STREAM family (64-bit offsets) at every batch size:
+    the workspace is that of the forced family."""
+    from vllm_xpu_kernels import capi
+    a = capi.FusedMoeArgs(recipe=recipe, activation=0, act_dtype=1, ids_dtype=3,
+                          num_tokens=tokens, hidden=hidden, inter=inter, num_experts=2, topk=1,
+                          w_layout=1, w_group=128, w13_scale=1, w2_scale=1)
+    got = lib.mi355moe_fused_moe_workspace_size(ctypes.byref(a))
+    monkeypatch.setenv("MI355MOE_GEMM_TILE", "small")  # (through the same check)
+    assert lib.mi355moe_fused_moe_workspace_size(ctypes.byref(a)) == got
+    monkeypatch.setenv("MI355MOE_GEMM_TILE", "stream")
+    assert lib.mi355moe_fused_moe_workspace_size(ctypes.byref(a)) == got
+
+
 @pytest.mark.parametrize("field,value,message", [
     ("num_tokens", -1, b"invalid layer shape"), ("topk", 0, b"invalid layer shape"),
     ("num_experts", 2048, b"at most 1024"), ("hidden", 7100, b"% 128"),

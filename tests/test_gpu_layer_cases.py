@@ -217,3 +217,33 @@ def test_fused_moe_ep(dev, recipe, dt, ep_rank, T):
     else:
         tol = 2e-2 if dt == torch.bfloat16 else 1e-2
         torch.testing.assert_close(got, ref, rtol=tol, atol=tol)
+
+
+def test_huge_expert_beyond_32_bit_offsets(dev):
+    """One bf16 expert of 2^31 w13 weights, more slots than the SMALL range:
+    the K-blocked layer streams it with 64-bit offsets (the SMALL kernel
+    refuses it).  Reference: fp32 products of the same 16-bit values, rounded
+    to bf16 where the layer rounds (w13's output, the activation, the
+    output): bf16 bar of this file."""
+    H = I = 32768
+    T = 150
+    print(f"huge expert: H={H} I={I} T={T}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(1)
+    w13 = torch.empty(1, H, 2 * I, dtype=torch.bfloat16, device=dev).normal_(0, 1, generator=g)
+    w2 = torch.empty(1, I, H, dtype=torch.bfloat16, device=dev).normal_(0, 1, generator=g)
+    w13.mul_(H ** -0.5)
+    w2.mul_(I ** -0.5)
+    x = torch.randn(T, H, generator=g, device=dev).to(torch.bfloat16)
+    step = 4096
+
+    def product(a, w):  # [T, K] @ [K, N], a few columns in fp32 at a time
+        return torch.cat([a.float() @ w[:, n:n + step].float()
+                          for n in range(0, w.shape[1], step)], 1).to(torch.bfloat16)
+    g1 = product(x, w13[0])
+    act = (torch.nn.functional.silu(g1[:, :I].float()) * g1[:, I:].float()).to(torch.bfloat16)
+    ref = product(act, w2[0]).float()
+    moe = _layer_cls()(w13, None, None, w2, None, None, 1, "silu", 1)
+    out = torch.empty_like(x)
+    moe.apply(out, x, torch.ones(T, 1, device=dev),
+              torch.zeros(T, 1, dtype=torch.int32, device=dev))
+    torch.testing.assert_close(out.float(), ref, rtol=2e-2, atol=2e-2)

@@ -553,10 +553,6 @@ FusedLayout plan_with(const mi355moe_fused_moe_args* a, uint8_t* base, int max_b
   if (a->expert_map && a->expert_map_len > E) local = cdiv(L.slots * E, a->expert_map_len);
   L.tile = pick_tile(gemm_recipe(a), wide_ok, L.slots, local, E, &L.bm);
   if (L.tile == TILE_WIDE && max_bm < kWideBM) L.tile = TILE_SMALL;
-  if (L.tile == TILE_SMALL && !(mid_fits(2 * I, H) && mid_fits(H, K2))) {
-    L.tile = TILE_STREAM;  // 64-bit weight offsets
-    L.bm = 16;
-  }
   // K-blocked weights: the families that read them (STREAM, SMALL, WIDE, and
   // BIG for fp8, whose 8-wave kernel takes K <= 8192, and for mxfp4)
   if (kblock && a->recipe != MI355MOE_RECIPE_MXFP4 &&
@@ -564,6 +560,11 @@ FusedLayout plan_with(const mi355moe_fused_moe_args* a, uint8_t* base, int max_b
       !(L.tile == TILE_BIG && a->recipe == MI355MOE_RECIPE_FP8BLOCK)) {
     L.tile = TILE_SMALL;
     L.bm = 64;
+  }
+  // after every route to SMALL: experts beyond its 32-bit weight offsets
+  if (L.tile == TILE_SMALL && !(mid_fits(2 * I, H) && mid_fits(H, K2))) {
+    L.tile = TILE_STREAM;  // 64-bit weight offsets
+    L.bm = 16;
   }
   if (L.tile == TILE_SMALL) L.bm = std::min(L.bm, max_bm);
   padded_sizes(L.slots, E, L.bm, L.max_padded, L.max_blocks);
