@@ -935,18 +935,20 @@ def test_fused_moe_int4(dev, dt, T, topk):
 @pytest.mark.parametrize("grp", [32, 128, 256])
 @pytest.mark.parametrize("T", [2, 64, 2048])
 @pytest.mark.parametrize("layout", ["kblock", "nk"])
-def test_fused_moe_int4_group_scales(dev, monkeypatch, grp, T, layout):
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_fused_moe_int4_group_scales(dev, monkeypatch, grp, T, layout, dt):
     """int4 with a different 16-bit scale in every (row, group) and random
     biases, against the oracle (64 sampled tokens): K-blocked weights and
     scales through the stream (T=2), small (T=64) and 320-slot (T=2048)
     kernels, where one group spans 1, 4 or 8 of the 320-slot kernel's
     32-value stages and the scales of a stage move with the weights; the
     row-major layout (MI355MOE_WEIGHT_LAYOUT=nk) through the stream, small
-    and 128-slot kernels."""
+    and 128-slot kernels.  fp16, K-blocked, T=64, groups of 128 and 256: the
+    16-slot blocks that scale the fp32 sums (a group a stage, a group over
+    two stages)."""
     from vllm_xpu_kernels.fused_moe_interface import XpuFusedMoe
     if layout == "nk":
         monkeypatch.setenv("MI355MOE_WEIGHT_LAYOUT", "nk")
-    dt = torch.bfloat16
     g = torch.Generator().manual_seed(31 + T + grp)
     E, H, I, topk = 16, 1024, 512, 2
     u13 = torch.randint(0, 0xff, (E, 2 * I, H // 2), generator=g).to(torch.uint8)
@@ -965,7 +967,8 @@ def test_fused_moe_int4_group_scales(dev, monkeypatch, grp, T, layout):
     toks = torch.linspace(0, T - 1, min(T, 64)).long()
     ref = O.fused_moe("int4", x[toks], u13 ^ 0x88, s13, b13, u2 ^ 0x88, s2, b2, tw[toks],
                       ti[toks])
-    torch.testing.assert_close(out.cpu()[toks], ref, rtol=2e-2, atol=2e-2)
+    tol = 2e-2 if dt == torch.bfloat16 else 1e-2
+    torch.testing.assert_close(out.cpu()[toks], ref, rtol=tol, atol=tol)
 
 
 def test_fused_moe_a1q_scale_rejected_outside_fp8block(dev):

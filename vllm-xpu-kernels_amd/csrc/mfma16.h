@@ -96,8 +96,10 @@ __device__ __forceinline__ uint4 fp8x8_to16(uint2 w) {
 // The nibbles with the sign bit flipped, u = v + 8, one to a byte, are the
 // e4m3 values u * 2^-9, which a scaled conversion turns into u, two per
 // instruction.  fp16: u - 8 and its product with the scale packed; bf16: u *
-// s - 8 * s in fp32 (exact: 4 + 8 bits), one rounding.  18 / 22 VALU per 8
-// values; a bit-field extract, conversion and product per value took 28.
+// s - 8 * s in fp32 (exact: 4 + 8 bits), one rounding; where 8 * s overflows
+// (code -8 is infinite then), the group's weights are infinite or NaN.  18 / 22
+// VALU per 8 values; a bit-field extract, conversion and product per value
+// took 28, u - 8 before the product for bf16 26 (4 % of a layer).
 template <bool F16>
 __device__ __forceinline__ uint4 int4x8_to16(uint32_t w, float sc) {
   const uint32_t t = w ^ 0x88888888u;

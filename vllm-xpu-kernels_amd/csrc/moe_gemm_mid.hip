@@ -49,7 +49,10 @@ __device__ __forceinline__ f32x4 mfma_e4m3(uint4 a0, uint4 a1, uint4 b0, uint4 b
 // v1 v3 v5 v7, in which the activation is staged too (even_odd); int4x8_to16,
 // which rounds every product, takes 18.  The -8 per weight is one MFMA per
 // step with a constant operand, shared by all weight rows.  16-slot blocks
-// only (61 tokens of Qwen3-30B: 87 -> 76 us; with 32 slots equal).
+// only (61 tokens of Qwen3-30B: 87 -> 76 us; with 32 slots equal).  Rounding
+// no weight, it is the closer to 64 bits (layer of 61 tokens: 5.2e-4 against
+// 6.0e-4); an infinite activation makes its slot's outputs NaN, where products
+// of single weights give infinities, and NaN for weights of 0.
 __device__ __forceinline__ uint4 int4x8_to_u16(uint32_t w) {
   const uint32_t t = w ^ 0x88888888u;
   const uint32_t lo = t & 0x0f0f0f0fu, hi = (t >> 4) & 0x0f0f0f0fu;
@@ -607,7 +610,10 @@ int launch_moe_gemm_mid(int recipe, int epi, bool qout, int bm, const GemmArgs& 
     case MI355MOE_RECIPE_INT4: {
       const bool rows = a.w_kblock && a.w_group % KB == 0 && a.ldb_rows % 4 == 0 &&
                         a.up_off % 4 == 0 && aligned(a.b_scale, 8);
-      if (rows && a.out_f16 && bm == 16)  // four rows' scales in one load, on the sums
+      // POST, four rows' scales in one load: the same call in larger blocks,
+      // row-major, or with scales off an 8-byte boundary rounds every weight
+      // (6e-4 apart, relative to the layer's output)
+      if (rows && a.out_f16 && bm == 16)
         return epi == EPI_GLU
                    ? launch_mid_t<MI355MOE_RECIPE_INT4, 1, EPI_GLU, false, true, false>(a, max_blocks, qs, st)
                    : launch_mid_t<MI355MOE_RECIPE_INT4, 1, EPI_STORE, false, true, false>(a, max_blocks, qs, st);
