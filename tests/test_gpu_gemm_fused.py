@@ -132,6 +132,12 @@ def test_grouped_gemm_mxfp4_zero_scale_code_is_zero(dev):
 
 
 # -------------------------------------------------------------- fused layer
+def _force(monkeypatch, tile):
+    """Run the named kernel family (None: the dispatch's own choice)."""
+    if tile:
+        monkeypatch.setenv("MI355MOE_GEMM_TILE", tile)
+
+
 def _layer(cfg, T, dev, E=None, seed_shift=0):
     """Build weights/inputs of `cfg` (optionally with E experts), route on
     the GPU, run XpuFusedMoe; return everything the oracle needs."""
@@ -215,16 +221,19 @@ def test_fused_moe_c3_full_size_every_token(dev):
     _close(out, _oracle_layer_on_device(cfg, w, x, tw, ti), fp8=True)
 
 
-@pytest.mark.parametrize("T", [1, 256, 2048, 8192])
-def test_fused_moe_fp8block_swigluoai_c3(dev, T):
+@pytest.mark.parametrize("T,tile", [(1, None), (256, None), (2048, None), (2048, "big"),
+                                    (8192, None)])
+def test_fused_moe_fp8block_swigluoai_c3(dev, monkeypatch, T, tile):
     """fp8 block-scaled weights with an interleaved swigluoai w13 (gate row
     2j, up row 2j + 1, 128 x 128 scale blocks) at the DeepSeek-V3 shape (256
     experts, H=7168, I=2048): the layer splits the rows into gate and up
     halves read with one scale row per 64 weight rows, through the decode
-    (T=1), small (T=256), 128-slot (T=2048) and 320-slot (T=8192) kernels;
-    every token against the oracle run on the device (interleaved rows, the
+    (T=1), small (T=256) and 320-slot (T=2048, 8192) kernels and the 128-slot
+    one, which the dispatch keeps for activations of 4 GiB and more; every
+    token against the oracle run on the device (interleaved rows, the
     reference's block scales), to the fp8 bar."""
     import dataclasses
+    _force(monkeypatch, tile)
     cfg = dataclasses.replace(_W().CONFIGS["C3"], activation="swigluoai")
     cfg, w, x, tw, ti, out, moe = _layer(cfg, T, dev)
     assert moe._ws_rows == 64 and moe.gemm1_wei_scales.shape[1] == 2 * cfg.inter // 64
@@ -284,9 +293,9 @@ BIG_ROWS = [300, 260, 0, 129]
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("recipe", ["bf16", "fp8block", "mxfp4"])
 def test_grouped_gemm_big_tiles(dev, recipe, dt):
-    """>96 rows per expert: bf16 and fp8 select the 320x256 kernels, mxfp4
-    the LDS-staged 128x256 one; N=2880 is not a multiple of the tile (ragged
-    last tile)."""
+    """172 rows per expert: bf16 and fp8 select the 320x256 kernels, mxfp4
+    (row-major) the LDS-staged 128x256 one; N=2880 is not a multiple of the
+    tile (ragged last tile)."""
     g = torch.Generator().manual_seed(4)
     E, K = 4, 1024
     N = 640 if recipe == "fp8block" else 2880
@@ -320,7 +329,7 @@ WIDE_ROWS = [1, 31, 33, 64, 97, 159, 160, 161, 255, 319, 320, 321, 700]
 @pytest.mark.parametrize("K", [32, 64, 96, 352])
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float16])
 def test_grouped_gemm_wide_tiles(dev, K, out_dtype):
-    """bf16 weights with >96 rows per expert select the 320x256 kernel.
+    """bf16 weights with more than 104 rows per expert select the 320x256 kernel.
     Valid rows per 320-slot block 1..320 (every count of 32-row MFMA groups
     per wave half, 0..5, and of skipped 16-row DMA groups; experts of 1, 2
     and 3 blocks); K from one 32-element stage (shorter than the 3-deep
@@ -358,8 +367,8 @@ W8_ROWS = [1, 15, 17, 64, 100, 159, 160, 161, 200, 319, 320, 321, 700, 1000, 120
 
 @pytest.mark.parametrize("K", [128, 384, 1024])
 def test_grouped_gemm_wide8_tiles(dev, K):
-    """fp8 block-scaled weights with >160 rows per expert select the 320x256
-    kernel.  Valid rows per 320-slot block 1..320 (every count of 16-slot
+    """fp8 block-scaled weights with more than 44 rows per expert select the
+    320x256 kernel.  Valid rows per 320-slot block 1..320 (every count of 16-slot
     MFMA tiles per wave half, 0..10, skipped 8-row DMA groups and 64-slot
     scale groups); experts of 1, 2 and 3 blocks; K from one 128-element
     stage (no DMA ahead) to 8; N=640 is two and a half 256-row tiles."""
@@ -376,20 +385,22 @@ def test_grouped_gemm_wide8_tiles(dev, K):
     torch.testing.assert_close(d.cpu().float(), ref.float(), rtol=1e-2, atol=1e-2)
 
 
-def test_grouped_gemm_big8_tiles(dev):
-    """fp8 block-scaled weights with 97..160 rows per expert select the
-    128x256 8-wave kernel (128-slot blocks; experts of 1 and 2 blocks, a
-    partial last block)."""
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_grouped_gemm_big8_tiles(dev, monkeypatch, dt):
+    """The 128x256 8-wave fp8 block-scaled kernel, which the dispatch keeps
+    for activations of 4 GiB and more (forced here): 128-slot blocks; experts
+    of 0, 1 and 2 blocks, a partial last block."""
+    _force(monkeypatch, "big")
     g = torch.Generator().manual_seed(13)
     rows_l = [129, 100, 150, 0, 201]
     E, N, K = len(rows_l), 384, 512
     M = sum(rows_l)
-    a = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    a = torch.randn(M, K, generator=g).to(dt)
     q, s = O.fp8_block_quant_weight(torch.randn(E, N, K, generator=g) * 0.02)
-    d = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=dev)
+    d = torch.full((M, N), float("nan"), dtype=dt, device=dev)
     _ops().cutlass_grouped_gemm(a.to(dev), q.to(dev), s.to(dev), None, d,
                                 torch.tensor(rows_l, dtype=torch.int32, device=dev), N, K, E)
-    ref = O.grouped_gemm("fp8block", a, q, s, None, rows_l)
+    ref = O.grouped_gemm("fp8block", a, q, s, None, rows_l, out_dtype=dt)
     torch.testing.assert_close(d.cpu().float(), ref.float(), rtol=1e-2, atol=1e-2)
 
 
@@ -413,7 +424,7 @@ def test_grouped_gemm_fp8_k_beyond_wide8(dev):
 def test_fused_moe_wide8_ragged(dev, T):
     """Whole fp8 block-scaled layer through the 320x256 kernels: the w13
     epilogue re-quantises the activation to e4m3 (1x128 groups) in LDS;
-    T=700 leaves about 175 slots per expert (second wave half nearly idle)."""
+    T=700 leaves about 175 slots per expert."""
     import dataclasses
     cfg = dataclasses.replace(_W().CONFIGS["C2"], recipe="fp8block", hidden=384, inter=256,
                               experts=8, topk=2)
@@ -450,11 +461,15 @@ def _layer_both_layouts(cfg, T, dev, monkeypatch):
     return res, out_nk
 
 
-@pytest.mark.parametrize("T", [1, 16, 256, 512, 1024, 2048])
-def test_fused_moe_kblock_equals_nk_c2(dev, monkeypatch, T):
+@pytest.mark.parametrize("T,tile", [(1, None), (16, None), (16, "stream"), (256, None),
+                                    (512, None), (1024, None), (1024, "wide"), (2048, None)])
+def test_fused_moe_kblock_equals_nk_c2(dev, monkeypatch, T, tile):
     """The K-blocked layout changes addresses only: every kernel family (T=1
-    split-K stream, 16 stream, 256/512 small, 1024/2048 wide) gives the
-    row-major layer's output bit for bit, and that output meets the oracle."""
+    split-K stream, 16 to 1024 small, in blocks of 16 to 96 slots, 2048 wide;
+    the stream and wide kernels also at sizes where the dispatch takes
+    small) gives the row-major layer's output bit for bit, and that output
+    meets the oracle."""
+    _force(monkeypatch, tile)
     (cfg, w, x, tw, ti, out, _), out_nk = _layer_both_layouts(_W().CONFIGS["C2"], T, dev,
                                                              monkeypatch)
     assert torch.equal(out, out_nk)
@@ -476,15 +491,17 @@ def test_fused_moe_kblock_ragged(dev, monkeypatch, activation, T):
 
 
 @pytest.mark.parametrize("activation", ["silu", "swigluoai"])
-@pytest.mark.parametrize("T", [8, 32, 48, 96, 500, 1024])
-def test_fused_moe_kblock_fp8_families(dev, monkeypatch, T, activation):
+@pytest.mark.parametrize("T,tile", [(8, None), (32, None), (48, None), (96, None),
+                                    (96, "big"), (500, None), (500, "big"), (1024, None)])
+def test_fused_moe_kblock_fp8_families(dev, monkeypatch, T, tile, activation):
     """fp8 block-scaled weights K-blocked in 128-byte blocks (H=384, I=256,
     8 experts, top-2: about T/4 slots per expert): stream (T=8), small
-    (32, 48), 128-slot 8-wave (96, 500) and 320-slot (1024) kernels each give
-    the row-major layer's output bit for bit, within the fp8 bar of the
-    oracle; swigluoai (interleaved rows, read as gate / up halves with
+    (32, 48, 96), 320-slot (500, 1024) and 128-slot 8-wave ("big") kernels
+    each give the row-major layer's output bit for bit, within the fp8 bar of
+    the oracle; swigluoai (interleaved rows, read as gate / up halves with
     64-row scale blocks) through the same kernels."""
     import dataclasses
+    _force(monkeypatch, tile)
     cfg = dataclasses.replace(_W().CONFIGS["C2"], recipe="fp8block", hidden=384, inter=256,
                               experts=8, topk=2, activation=activation)
     (cfg, w, x, tw, ti, out, _), out_nk = _layer_both_layouts(cfg, T, dev, monkeypatch)
@@ -512,7 +529,7 @@ def test_pack_mxfp4_kblock_layout(dev, shape):
 def test_fused_moe_kblock_mxfp4_families(dev, monkeypatch, T):
     """mxfp4 weights and e8m0 scales K-blocked (32-value blocks; H=320,
     I=256, swigluoai with biases, 8 experts, top-2): stream (T=8) and small
-    (96: 16-slot blocks, 160: 32-slot blocks) kernels give the row-major
+    (96: 32-slot blocks, 160: 64-slot blocks) kernels give the row-major
     layer's output bit for bit, within the bar of the oracle."""
     import dataclasses
     cfg = dataclasses.replace(_W().CONFIGS["C5"], hidden=320, inter=256, experts=8, topk=2)
@@ -532,7 +549,7 @@ def _assert_near_layouts(out, out_nk):
 @pytest.mark.parametrize("shape", [(320, 256, 1024), (320, 256, 2000), (352, 160, 700),
                                    (96, 64, 1200)])
 def test_fused_moe_mxfp4_wide(dev, monkeypatch, shape):
-    """K-blocked mxfp4 layers whose experts average > 96 slots run the
+    """K-blocked mxfp4 layers whose experts average > 130 slots run the
     320-slot mxfp4 kernel (row-major weights: the 128-slot register-staged
     one): H=320 / I=256 (10 and 8 K stages), H=352 / I=160 (11 and 5 K
     stages: GLU and STORE tiles with columns past N), H=96 / I=64 (K loops
@@ -574,15 +591,17 @@ def test_fused_moe_mxfp4_wide_skewed(dev, hot):
     _close(out[toks], _oracle_layer(cfg, w, x, tw, ti, toks))
 
 
-@pytest.mark.parametrize("T", [1, 16, 48, 300, 1024])
-def test_fused_moe_a1q_scale_pre_quantised(dev, T):
+@pytest.mark.parametrize("T,tile", [(1, None), (16, None), (16, "stream"), (48, None),
+                                    (300, None), (300, "big"), (1024, None)])
+def test_fused_moe_a1q_scale_pre_quantised(dev, monkeypatch, T, tile):
     """Pre-quantised hidden states (a1q_scale, fp8block; H=384, I=256, 8
     experts, top-2): the (q, s) of the layer's own 1x128 quantiser give its
-    bf16-input output bit for bit in every family (T=1 split-K stream, 16
-    stream, 48 small, 300 128-slot, 1024 320-slot); other scales (ue8m0)
-    meet the oracle run on the same pre-quantised input."""
+    bf16-input output bit for bit in every family (T=1 split-K stream, 16 and
+    48 small, 300 and 1024 320-slot; stream and 128-slot forced); other scales
+    (ue8m0) meet the oracle run on the same pre-quantised input."""
     import dataclasses
     from vllm_xpu_kernels import ops
+    _force(monkeypatch, tile)
     cfg = dataclasses.replace(_W().CONFIGS["C2"], recipe="fp8block", hidden=384, inter=256,
                               experts=8, topk=2)
     cfg, w, x, tw, ti, out, moe = _layer(cfg, T, dev)
@@ -642,15 +661,19 @@ def test_fused_moe_generic_activation_clamp(dev):
         _close(out, ref)
 
 
-@pytest.mark.parametrize("recipe", ["bf16", "fp8block", "mxfp4", "mxfp8"])
-@pytest.mark.parametrize("T", [1, 16, 48, 300, 1024])
-def test_fused_moe_fp16(dev, recipe, T):
+@pytest.mark.parametrize("recipe,T,tile", [
+    *((r, T, None) for r in ("bf16", "fp8block", "mxfp4", "mxfp8")
+      for T in (1, 16, 48, 300, 1024)),
+    *((r, 16, "stream") for r in ("bf16", "fp8block", "mxfp4")), ("fp8block", 300, "big")])
+def test_fused_moe_fp16(dev, monkeypatch, recipe, T, tile):
     """fp16 hidden states, output and biases (16-bit recipe: fp16 weights;
     mxfp4 dequantised to fp16) through every kernel family (H=384, I=256, 8
-    experts, top-2; T=1 split-K stream ... 1024 320-slot), at the reference's
-    fp16 bar rtol = atol = 1e-2 (tests/fused_moe/test_fused_moe.py:288-294;
-    fp8 at its own bar).  mxfp4 runs swigluoai with biases, the others SiLU."""
+    experts, top-2; T=1 split-K stream ... 1024 320-slot; stream and the fp8
+    128-slot kernel forced), at the reference's fp16 bar rtol = atol = 1e-2
+    (tests/fused_moe/test_fused_moe.py:288-294; fp8 at its own bar).  mxfp4
+    runs swigluoai with biases, the others SiLU."""
     import dataclasses
+    _force(monkeypatch, tile)
     from vllm_xpu_kernels.fused_moe_interface import XpuFusedMoe
     W = _W()
     cfg = dataclasses.replace(W.CONFIGS["C5" if recipe == "mxfp4" else "C2"], recipe=recipe,
@@ -1043,10 +1066,12 @@ def test_fused_moe_mxfp4_pre_quantised_w4a4(dev, T, dt):
     assert (out4.float() - out.float()).abs().mean() < 0.25 * out.float().abs().mean()
 
 
-@pytest.mark.parametrize("T", [1, 16])
-def test_fused_moe_kblock_fp8_c3_decode(dev, monkeypatch, T):
-    """DeepSeek-V3 shapes at decode (split-K stream kernels): K-blocked and
-    row-major fp8 weights give the same layer output bit for bit."""
+@pytest.mark.parametrize("T,tile", [(1, None), (16, None), (16, "stream")])
+def test_fused_moe_kblock_fp8_c3_decode(dev, monkeypatch, T, tile):
+    """DeepSeek-V3 shapes at decode (T=1 split-K stream, 16 small and stream
+    kernels): K-blocked and row-major fp8 weights give the same layer output
+    bit for bit."""
+    _force(monkeypatch, tile)
     (cfg, w, x, tw, ti, out, _), out_nk = _layer_both_layouts(_W().CONFIGS["C3"], T, dev,
                                                              monkeypatch)
     assert torch.equal(out, out_nk)

@@ -5,8 +5,8 @@
   clamp a large share of gate/up values; SiLU as the reference, plus
   swigluoai (interleaved G1, where the reference's column-half clamp falls on
   both gate and up of the first I/2 pairs) and a limit that is not a bf16
-  value.  Token counts cover the split-K STREAM, STREAM, SMALL and 128/320-slot
-  kernels.
+  value.  Token counts cover the split-K STREAM, STREAM, SMALL and 320-slot
+  kernels; the 128-slot ones are forced.
 * expert parallelism (reference :534-909): E = 16 global experts, ep_size 4,
   the layer built on one rank's 4 experts with ep_rank / ep_size, for the
   16-bit, per-expert fp8, int4, mxfp4 and fp8block recipes.
