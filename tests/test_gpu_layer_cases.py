@@ -219,6 +219,43 @@ def test_fused_moe_ep(dev, recipe, dt, ep_rank, T):
         torch.testing.assert_close(got, ref, rtol=tol, atol=tol)
 
 
+@pytest.mark.parametrize("recipe,dt", [("bf16", torch.bfloat16), ("fp8", torch.bfloat16),
+                                       ("int4", torch.float16), ("mxfp4", torch.bfloat16),
+                                       ("fp8block", torch.bfloat16)])
+@pytest.mark.parametrize("T", [20, 130])
+@pytest.mark.parametrize("route", ["all here", "one expert", "none here"])
+def test_fused_moe_ep_share_off(dev, recipe, dt, T, route):
+    """Expert parallelism whose routing is not the even share that the block
+    size is chosen by (5 and 32 slots per expert: 16- to 64-slot blocks): every
+    slot on this rank's experts (four times the share), every token's one
+    local slot on one expert, and no local slot at all."""
+    print(f"EP share off: {recipe} {dt} T={T} {route}", flush=True)
+    g = torch.Generator().manual_seed(3 + T)
+    H, I, topk = 256, 256, 4
+    lay, ora = _ep_weights(recipe, dt, g, H, I)
+    e = E_GLOBAL // EP_SIZE
+    lo, hi = e, 2 * e
+    x = (torch.randn(T, H, generator=g) / 16).to(dt)
+    tw = torch.rand(T, topk, generator=g)
+    far = torch.stack([torch.randperm(E_GLOBAL - 2 * e, generator=g)[:topk] for _ in range(T)]) + hi
+    ti = {"all here": torch.stack([torch.randperm(e, generator=g) for _ in range(T)]) + lo,
+          "one expert": torch.cat([torch.full((T, 1), lo + 1), far[:, 1:]], 1),
+          "none here": far}[route]
+    loc = [None if t is None else t[lo:hi].contiguous().to(dev) for t in lay]
+    moe = _layer_cls()(*loc, topk, "silu", e, ep_rank=1, ep_size=EP_SIZE)
+    out = torch.full((T, H), float("nan"), dtype=dt, device=dev)
+    moe.apply(out, x.to(dev), tw.to(dev), ti.to(dev))
+    ref = O.fused_moe(recipe, x, *[None if t is None else t[lo:hi] for t in ora], tw, ti,
+                      expert_map=O.init_expert_map(e, 1, EP_SIZE))
+    if route == "none here":
+        assert torch.all(out == 0)
+    elif recipe == "fp8block":
+        _close_fp8(out.cpu(), ref)
+    else:
+        tol = 2e-2 if dt == torch.bfloat16 else 1e-2
+        torch.testing.assert_close(out.cpu(), ref, rtol=tol, atol=tol)
+
+
 def test_huge_expert_beyond_32_bit_offsets(dev):
     """One bf16 expert of 2^31 w13 weights, more slots than the SMALL range:
     the K-blocked layer streams it with 64-bit offsets (the SMALL kernel
