@@ -484,6 +484,30 @@ def test_fused_moe_huge_experts_stream(lib, monkeypatch, recipe, hidden, inter, 
     assert lib.mi355moe_fused_moe_workspace_size(ctypes.byref(a)) == got
 
 
+@pytest.mark.parametrize("kw,ranks,wide", [
+    # fp8 block-scaled, a rank of 8: 18 slots per expert by its share of all
+    # tokens' slots, 35 where every token has one here; then 31 and 59
+    (dict(recipe=1, num_tokens=600, hidden=7168, inter=2048, num_experts=32), 8, False),
+    (dict(recipe=1, num_tokens=1003, hidden=7168, inter=2048, num_experts=32), 8, True),
+    # bf16, a rank of 4: 71 and 98; 94 and 129
+    (dict(recipe=0, num_tokens=1150, hidden=2048, inter=768, num_experts=32), 4, False),
+    (dict(recipe=0, num_tokens=1500, hidden=2048, inter=768, num_experts=32), 4, True),
+    # int4 keeps to the share: 93
+    (dict(recipe=3, num_tokens=1500, hidden=2048, inter=768, num_experts=16, w_group=128), 8,
+     False)])
+def test_fused_moe_expert_map_family(lib, monkeypatch, kw, ranks, wide):
+    """Expert parallelism: whether a layer takes the 320-slot kernels, by the
+    slots of tokens that a dispatch sent here (the workspace is then that of
+    the forced family)."""
+    from vllm_xpu_kernels import capi
+    a = capi.FusedMoeArgs(activation=0, act_dtype=1, ids_dtype=3, topk=8, w_layout=1,
+                          w13_scale=1, w2_scale=1, expert_map=64,
+                          expert_map_len=ranks * kw["num_experts"], **kw)
+    got = lib.mi355moe_fused_moe_workspace_size(ctypes.byref(a))
+    monkeypatch.setenv("MI355MOE_GEMM_TILE", "wide")
+    assert (lib.mi355moe_fused_moe_workspace_size(ctypes.byref(a)) == got) == wide
+
+
 @pytest.mark.parametrize("field,value,message", [
     ("num_tokens", -1, b"invalid layer shape"), ("topk", 0, b"invalid layer shape"),
     ("num_experts", 2048, b"at most 1024"), ("hidden", 7100, b"% 128"),

@@ -546,11 +546,31 @@ FusedLayout plan_with(const mi355moe_fused_moe_args* a, uint8_t* base, int max_b
   const bool kblock = a->w_layout == MI355MOE_WLAYOUT_KBLOCK;
   const bool wide_ok = wide_ok_for(gemm_recipe(a), a->num_tokens, 2 * I, H, kblock) &&
                        wide_ok_for(gemm_recipe(a), L.slots + E * kWideBM, H, K2, kblock);
-  // expert parallelism: of the slots routed over expert_map_len experts this
-  // rank's E take their share (rank of 8 of DeepSeek-V3, 1003 tokens: 31 slots
-  // per expert, not 251; the 320-slot kernel took 332 us, 64-slot blocks 297)
+  // Expert parallelism.  A call with every rank's tokens brings this rank's E
+  // of expert_map_len experts their share of the slots; one with the tokens
+  // that a dispatch sent here, up to two per token on a rank of 8 (`here`: one
+  // slot of a token is here, its others spread evenly).  The host cannot tell
+  // them apart, so blocks are sized by the share only where the larger count
+  // does not cost more than it saves:
+  //   fp8 block-scaled, by `here`: blocks that overflow stream the weights twice.
+  //     Rank of 8 of DeepSeek-V3, us at the share / 1.5 / 2 / 3 times it, by the
+  //     share | by `here`: 600 tokens 264 317 403 467 | 270 272 278 355; 1003
+  //     tokens 287 296 410 445 | 299 306 314 330; 1350 tokens 299 425 438 577 |
+  //     307 320 330 346 (all slots taken as local: 323 to 381)
+  //   bf16, by `here` above 72 slots per expert (SMALL or WIDE): rank of 4 of
+  //     Qwen3-30B, 1500 tokens, at half / 1 / 1.5 times: 86 96 140 | 81 90 99; below,
+  //     by the share: rank of 8, 740 tokens, 1 / 1.5 / 2 / 3: 50 59 57 73 | 55 60 63 78
+  //   int4 (rank of 8 of Qwen3-30B, 1500 tokens 69 73 79 104 | 107 116 124 143),
+  //     mxfp4 and per-expert fp8 by the share
   int64_t local = L.slots;
-  if (a->expert_map && a->expert_map_len > E) local = cdiv(L.slots * E, a->expert_map_len);
+  if (a->expert_map && a->expert_map_len > E) {
+    const int64_t share = cdiv(L.slots * E, a->expert_map_len);
+    const int64_t here = std::min(
+        L.slots, a->num_tokens + cdiv((L.slots - a->num_tokens) * E, a->expert_map_len));
+    const bool by_here = a->recipe == MI355MOE_RECIPE_FP8BLOCK ||
+                         (a->recipe == MI355MOE_RECIPE_BF16 && share > 72 * E);
+    local = by_here ? here : share;
+  }
   L.tile = pick_tile(gemm_recipe(a), wide_ok, L.slots, local, E, &L.bm);
   if (L.tile == TILE_WIDE && max_bm < kWideBM) L.tile = TILE_SMALL;
   // K-blocked weights: the families that read them (STREAM, SMALL, WIDE, and
