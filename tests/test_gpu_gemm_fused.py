@@ -525,11 +525,11 @@ def test_pack_mxfp4_kblock_layout(dev, shape):
     assert torch.equal(ps, sc.permute(0, 2, 1))
 
 
-@pytest.mark.parametrize("T", [8, 96, 160])
+@pytest.mark.parametrize("T", [8, 96, 160, 190])
 def test_fused_moe_kblock_mxfp4_families(dev, monkeypatch, T):
     """mxfp4 weights and e8m0 scales K-blocked (32-value blocks; H=320,
     I=256, swigluoai with biases, 8 experts, top-2): stream (T=8) and small
-    (96: 32-slot blocks, 160: 64-slot blocks) kernels give the row-major
+    (96, 160: 32-slot blocks, 190: 64-slot blocks) kernels give the row-major
     layer's output bit for bit, within the bar of the oracle."""
     import dataclasses
     cfg = dataclasses.replace(_W().CONFIGS["C5"], hidden=320, inter=256, experts=8, topk=2)
