@@ -229,7 +229,7 @@ def test_fused_moe_fp8block_swigluoai_c3(dev, monkeypatch, T, tile):
     experts, H=7168, I=2048): the layer splits the rows into gate and up
     halves read with one scale row per 64 weight rows, through the decode
     (T=1), small (T=256) and 320-slot (T=2048, 8192) kernels and the 128-slot
-    one, which the dispatch keeps for activations of 4 GiB and more; every
+    one, which the dispatch keeps for grouped GEMMs and huge batches; every
     token against the oracle run on the device (interleaved rows, the
     reference's block scales), to the fp8 bar."""
     import dataclasses
@@ -367,7 +367,7 @@ W8_ROWS = [1, 15, 17, 64, 100, 159, 160, 161, 200, 319, 320, 321, 700, 1000, 120
 
 @pytest.mark.parametrize("K", [128, 384, 1024])
 def test_grouped_gemm_wide8_tiles(dev, K):
-    """fp8 block-scaled weights with more than 44 rows per expert select the
+    """fp8 block-scaled weights with more than 96 rows per expert select the
     320x256 kernel.  Valid rows per 320-slot block 1..320 (every count of 16-slot
     MFMA tiles per wave half, 0..10, skipped 8-row DMA groups and 64-slot
     scale groups); experts of 1, 2 and 3 blocks; K from one 128-element
@@ -386,13 +386,14 @@ def test_grouped_gemm_wide8_tiles(dev, K):
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
-def test_grouped_gemm_big8_tiles(dev, monkeypatch, dt):
-    """The 128x256 8-wave fp8 block-scaled kernel, which the dispatch keeps
-    for activations of 4 GiB and more (forced here): 128-slot blocks; experts
-    of 0, 1 and 2 blocks, a partial last block."""
-    _force(monkeypatch, "big")
+@pytest.mark.parametrize("rows_l,tile", [([129, 100, 150, 0, 201], "big"),
+                                         ([129, 60, 1, 0, 128], None)])
+def test_grouped_gemm_big8_tiles(dev, monkeypatch, dt, rows_l, tile):
+    """The 128x256 8-wave fp8 block-scaled kernel, forced and as the dispatch
+    takes it (63 rows per expert, few columns): 128-slot blocks; experts of 0,
+    1 and 2 blocks, full and partial last blocks, one of a single row."""
+    _force(monkeypatch, tile)
     g = torch.Generator().manual_seed(13)
-    rows_l = [129, 100, 150, 0, 201]
     E, N, K = len(rows_l), 384, 512
     M = sum(rows_l)
     a = torch.randn(M, K, generator=g).to(dt)

@@ -1243,6 +1243,17 @@ GGLayout gg_plan(int recipe, bool need_quant, int64_t M, int64_t N, int64_t K, i
                  uint8_t* base) {
   int bm;
   GemmTile tile = pick_tile(recipe, wide_ok_for(recipe, M, 0, K), M, M, E, &bm);
+  // Without the position-ordered scales of a layer the 320-slot kernel reads
+  // one line per row and stage for each column tile; with few column tiles and
+  // up to 96 rows per expert the 128-slot kernel is the faster (320-slot ->
+  // 128-slot, us; 128 experts of 1536 x 2048, 52 rows 137 -> 124, 70 141 -> 130, 90
+  // 149 -> 133, 104 152 -> 162; 64 of 3072 x 4096, 52 to 90 rows: within the spread
+  // of runs; 32 of 7168 x 2048, 70 rows 127 -> 136)
+  if (tile == TILE_WIDE && recipe == MI355MOE_RECIPE_FP8BLOCK && N <= 3072 &&
+      M <= 96 * std::min(M, E) && !getenv("MI355MOE_GEMM_TILE")) {
+    tile = TILE_BIG;
+    bm = 128;
+  }
   if (tile == TILE_SMALL && !mid_fits(N, K)) {
     tile = TILE_STREAM;  // 64-bit weight offsets
     bm = 16;

@@ -1,9 +1,10 @@
 // Prefill grouped GEMM for fp8 e4m3 weights with 128x128 block scales and
 // e4m3 activations with 1x128 scales: 128-slot x 256-weight-row tiles, 8
 // waves, 3-slot LDS ring fed by direct global->LDS DMA.  The member of the
-// fp8 prefill family for calls whose activations are 4 GiB or more, which the
-// 320-slot kernel's 32-bit offsets do not reach: a 48.5 KB stage keeps two
-// stages of DMA in flight.
+// fp8 prefill family for grouped GEMMs of up to 3072 columns and 96 rows per
+// expert, and for calls whose activations are 4 GiB or more, which the 320-slot
+// kernel's 32-bit offsets do not reach: a 48.5 KB stage keeps two stages of DMA
+// in flight.
 //
 // Waves.  Eight waves, two per SIMD (waves w and w + 4 share SIMD w % 4), each
 // owning 64 slots x 64 weight rows: 4 x 4 tiles of the 16x16x128 e4m3 MFMA
