@@ -275,8 +275,9 @@ int launch_tile_gemm(GemmTile tile, int bm, int recipe, int epi, bool qout,
                      const GemmArgs& a, int64_t max_blocks, void* qs,
                      hipStream_t st);
 
-// Blocks of bm (16, 32, 64, 96 or 128) slots, every recipe but the MX ones
-// (moe_gemm_mid.hip), for experts of fewer than 2^30 weights (mid_fits).
+// Blocks of bm (16, 32, 64 or 96, for 16-bit and per-expert fp8 weights also 128)
+// slots, every recipe but the MX ones (moe_gemm_mid.hip), for experts of fewer
+// than 2^30 weights (mid_fits).
 bool mid_fits(int64_t ldb_rows, int64_t K);
 int launch_moe_gemm_mid(int recipe, int epi, bool qout, int bm, const GemmArgs& a,
                         int64_t max_blocks, void* qs, hipStream_t st);

@@ -100,7 +100,7 @@ GemmTile pick_tile(int recipe, bool wide_ok, int64_t slots, int64_t local, int64
   if (force >= 0 && !is_mx_recipe(recipe) && !is_w8a16_recipe(recipe)) {
     t = static_cast<GemmTile>(force);
     if (t == TILE_WIDE && !wide_ok) t = TILE_BIG;
-    b = t == TILE_STREAM ? 16 : t == TILE_WIDE ? kWideBM : t == TILE_SMALL && sb ? sb : 128;
+    b = t == TILE_STREAM ? 16 : t == TILE_WIDE ? kWideBM : t == TILE_SMALL ? (sb ? sb : 64) : 128;
   }
   *bm = b;
   return t;

@@ -21,6 +21,7 @@
 // tokens 332 -> 297, int4 Qwen3-30B fp16 61 tokens 150 -> 76, mxfp4
 // gpt-oss-20b 400 tokens 280 -> 156.
 #include <algorithm>
+#include <string>
 
 #include "mfma16.h"
 #include "moe_gemm.h"
@@ -569,9 +570,14 @@ int launch_mid(int bm, const GemmArgs& a, int64_t max_blocks, void* qs, hipStrea
     case 32: return launch_mid_t<RECIPE, 2, EPI, QOUT, false, GSC>(a, max_blocks, qs, st);
     case 64: return launch_mid_t<RECIPE, 4, EPI, QOUT, false, GSC>(a, max_blocks, qs, st);
     case 96: return launch_mid_t<RECIPE, 6, EPI, QOUT, false, GSC>(a, max_blocks, qs, st);
-    case 128: return launch_mid_t<RECIPE, 8, EPI, QOUT, false, GSC>(a, max_blocks, qs, st);
-    default: return set_error(MI355MOE_ERR_INVALID, "block_m must be 16, 32, 64, 96 or 128");
+    case 128:  // 16-bit and per-expert fp8 weights only (small_block)
+      if constexpr (RECIPE == MI355MOE_RECIPE_BF16 || is_w8a16_recipe(RECIPE))
+        return launch_mid_t<RECIPE, 8, EPI, QOUT, false, GSC>(a, max_blocks, qs, st);
+      break;
+    default: break;
   }
+  return set_error(MI355MOE_ERR_INVALID, "no SMALL kernel of this recipe for blocks of " +
+                                             std::to_string(bm) + " slots");
 }
 
 bool aligned(const void* p, uintptr_t n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) == 0; }
