@@ -10,8 +10,10 @@ namespace mi355 {
 namespace {
 // Block size of the SMALL family by the expected slots per active expert, 0:
 // beyond its range.  A block holds avg + 3 to 4 standard deviations where
-// the padded block is cheap, so that an expert's weights stream once; beyond
-// that larger blocks cost waves per SIMD.  us per layer, MI355X (block: 16 /
+// the padded block is cheap, so that most experts' weights stream once; beyond
+// that larger blocks cost waves per SIMD.  Lines lie at a measured minimum, or
+// 2 to 4 % beside it: bf16 16 (32 slots, 64 measured 230), int4 25 (64) and 125
+// (W), w8a16 94 (96), each seen on one shape only.  us per layer, MI355X (block: 16 /
 // 32 / 64 / 96 / 128, W the 320-slot kernel, - not measured):
 //   bf16  Qwen3-30B   avg 4: 213 221 218 229 234   16: 247 234 230 238 244
 //                     37: 351 302 251 255 262      56: 435 323 276 262 268 W 291

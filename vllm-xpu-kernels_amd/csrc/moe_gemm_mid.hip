@@ -9,17 +9,17 @@
 // is loaded two stages ahead into VGPRs and written one stage ahead to a
 // two-slot LDS buffer that all waves read as the MFMA's B operand: one
 // barrier a stage.  Four-wave workgroups and one stage in registers keep
-// three to eight waves on a SIMD, which hides the memory latency better than
-// more stages in fewer waves did (two and four stages measured 3 to 10 %
-// slower).  Loads are unconditional, from addresses limited to the expert's
+// two (96 and 128 slots) to eight waves on a SIMD (bf16: 3.9 / 3.3 resident at
+// 64 / 256 tokens of Qwen3-30B, fp8 5.5 at 64 of DeepSeek-V3), which hides the
+// memory latency better than more stages in fewer waves did (two and four
+// stages measured 3 to 10 % slower).  Loads are unconditional, from addresses limited to the expert's
 // range (a load under a branch makes the compiler wait for all loads in
 // flight where the branches join); what lies past K is zeroed before use.
 //
 // Measured per layer against the kernel before (one MFMA tile family, a wait
-// for the whole stage): bf16 Qwen3-30B 250 tokens 247 -> 227 us (of 1.2 GB:
-// 5.3 TB/s), fp8 DeepSeek-V3 512 tokens 2375 -> 1966, a rank of 8 with 1003
-// tokens 332 -> 297, int4 Qwen3-30B fp16 61 tokens 150 -> 76, mxfp4
-// gpt-oss-20b 400 tokens 280 -> 156.
+// for the whole stage): bf16 Qwen3-30B 250 tokens 247 -> 233 us (w13 141 us,
+// 5.8 TB/s), fp8 DeepSeek-V3 512 tokens 2375 -> 1966, int4 Qwen3-30B fp16 61
+// tokens 151 -> 76, mxfp4 gpt-oss-20b 400 tokens 280 -> 156.
 #include <algorithm>
 #include <string>
 
