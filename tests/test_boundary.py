@@ -508,6 +508,20 @@ def test_fused_moe_expert_map_family(lib, monkeypatch, kw, ranks, wide):
     assert (lib.mi355moe_fused_moe_workspace_size(ctypes.byref(a)) == got) == wide
 
 
+@pytest.mark.parametrize("recipe,hidden_scale", [(4, None), (4, 64), (2, 64)])
+def test_fused_moe_expert_map_mx_family(lib, recipe, hidden_scale):
+    """MX recipes (mxfp8; mxfp4 with e2m1 tokens) plan an expert-parallel layer
+    as without a map, by all slots: 300 tokens, 75 slots per expert of a rank of
+    8, its share 9 of them."""
+    from vllm_xpu_kernels import capi
+    a = capi.FusedMoeArgs(recipe=recipe, activation=0, act_dtype=1, ids_dtype=3, num_tokens=300,
+                          hidden=7168, inter=2048, num_experts=32, topk=8, w_layout=1,
+                          w13_scale=1, w2_scale=1, hidden_scale=hidden_scale)
+    whole = lib.mi355moe_fused_moe_workspace_size(ctypes.byref(a))
+    a.expert_map, a.expert_map_len = 64, 256
+    assert lib.mi355moe_fused_moe_workspace_size(ctypes.byref(a)) == whole
+
+
 @pytest.mark.parametrize("field,value,message", [
     ("num_tokens", -1, b"invalid layer shape"), ("topk", 0, b"invalid layer shape"),
     ("num_experts", 2048, b"at most 1024"), ("hidden", 7100, b"% 128"),

@@ -562,8 +562,11 @@ FusedLayout plan_with(const mi355moe_fused_moe_args* a, uint8_t* base, int max_b
   //     by the share: rank of 8, 740 tokens, 1 / 1.5 / 2 / 3: 50 59 57 73 | 55 60 63 78
   //   int4 (rank of 8 of Qwen3-30B, 1500 tokens 69 73 79 104 | 107 116 124 143),
   //     mxfp4 and per-expert fp8 by the share
+  //   MX recipes by all slots: below 17 slots per expert they stream the weights
+  //     once per 16 slots (mxfp8, rank of 8 of DeepSeek-V3, 300 / 520 tokens by the
+  //     share 404 441 512 636 / 457 547 727 929, by all 294 296 292 291 / 299 304 300 307)
   int64_t local = L.slots;
-  if (a->expert_map && a->expert_map_len > E) {
+  if (a->expert_map && a->expert_map_len > E && !mx_layer(a)) {
     const int64_t share = cdiv(L.slots * E, a->expert_map_len);
     const int64_t here = std::min(
         L.slots, a->num_tokens + cdiv((L.slots - a->num_tokens) * E, a->expert_map_len));
